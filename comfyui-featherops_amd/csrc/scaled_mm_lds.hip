@@ -14,9 +14,23 @@
 //     The swizzle is applied on the global side: the lane that fills LDS chunk
 //     p of row r fetches logical chunk p ^ swz(r);
 //   * three LDS stage buffers with two stages of copies in flight behind the
-//     one being multiplied (the split-K tiles: five or six buffers, four or
-//     five stages in flight); each barrier is preceded by an explicit vmcnt
+//     one being multiplied (the split-K tiles: four or five buffers, all but
+//     one in flight); each barrier is preceded by an explicit vmcnt
 //     wait that leaves the younger stages' copies in flight;
+//   * K groups (the split-K tiles): those tiles have one workgroup per CU, and
+//     with four waves, one per SIMD, nothing ran while a wave waited at a stage
+//     barrier or for its operands (M=2048 N=2048 on 64-row tiles: copies alone
+//     0.28 us a stage pair, MFMAs and operand reads alone 0.49, both 0.48-0.53).
+//     Two groups of four waves now share a stage of 128 K, each multiplying its
+//     own 64 for the whole tile, so that every SIMD has two waves and there is one
+//     barrier per 128 K; the groups' sums meet once, through LDS, after the
+//     last stage. Back to back, one group on a five- or six-stage ring -> two:
+//     M=154 N=10240 K=4096 21.3 -> 17.3 us, M=333 N=K=3072 15.7 -> 13.2, M=256
+//     N=K=3072 11.7 -> 9.9, M=512 N=3072 K=12288 47.7 -> 42.4, M=128 N=K=5120
+//     14.5 -> 13.3, M=77 N=K=4096 11.5 -> 9.6, M=64 N=13824 K=5120 22.1 ->
+//     20.6, M=256 N=K=1024 5.5 -> 5.3. Four groups on 64 x 64 (16 waves): 10.6
+//     at M=256 N=K=3072; 2 x 4 waves instead of two groups: 64 x 128 18.1 at
+//     M=154, and more LDS reads per MFMA;
 //   * per stage, the K halves are processed one after the other (all M
 //     repeats of K half 0, then of K half 1), so only half of the widened B
 //     operands are live at a time;
@@ -64,28 +78,35 @@ constexpr int kBK = 64;
 
 // kLora: 0 = none, 1 = fp16 factors, 2 = bf16 factors (T is M x R, U is N x R,
 // both row-major with R % 32 == 0 and 16-byte aligned rows)
-template <int BM, int BN, int WAVES_M, int WAVES_N, int kPipe, bool kBf16, bool kE4m3, int kLora, int kStages>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
+// kGroups: 1, or 2 = two groups of WAVES_M x WAVES_N waves share a stage of 2 x
+// 64 K, each multiplying its own 64 of it for the whole tile (see the K groups
+// paragraph in the file header). kTail: K need not be a multiple of the stage
+template <int BM, int BN, int WAVES_M, int WAVES_N, int kPipe, bool kBf16, bool kE4m3, int kLora, int kStages,
+          int kGroups, bool kTail>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_lds_kernel(
     const uint16_t* __restrict__ A, const uint8_t* __restrict__ Bp, const float* __restrict__ scale,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M, int N, int K, int has_scale, int has_bias,
     int tiles_m, int tiles_n, int group_m, int ksplit, float* __restrict__ partials, uint32_t* __restrict__ counters,
     const uint16_t* __restrict__ lora_t, const uint16_t* __restrict__ lora_u, int lora_rank, int c_nontemporal) {
-    constexpr int kWaves = WAVES_M * WAVES_N;
+    constexpr int kGroupWaves = WAVES_M * WAVES_N;
+    constexpr int kWaves = kGroupWaves * kGroups;
     constexpr int WTM = BM / WAVES_M;
     constexpr int WTN = BN / WAVES_N;
     constexpr int RM = WTM / 16;
     constexpr int RN = WTN / 16;
     static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be a multiple of 16");
-    constexpr int kAStage = BM * kBK * 2;
-    constexpr int kBStage = BN * kBK;
+    constexpr int kSK = kBK * kGroups;  // K per stage
+    constexpr int kASub = BM * kBK * 2;  // one group's share of a stage
+    constexpr int kBSub = BN * kBK;
+    constexpr int kAStage = kASub * kGroups;
+    constexpr int kBStage = kBSub * kGroups;
     constexpr int kStage = kAStage + kBStage;
     constexpr int kAInst = kAStage / 1024;  // 1 KB wave copies per stage
     constexpr int kBInst = kBStage / 1024;
-    static_assert(kAInst % kWaves == 0, "A copies must split evenly over waves");
-    constexpr int kAPerWave = kAInst / kWaves;
-    // B copies are rounded up to a whole number per wave; the surplus slots
-    // repeat the last copy (same bytes to the same LDS address), so every
+    // A and B copies are rounded up to a whole number per wave; the surplus
+    // slots repeat the last copy (same bytes to the same LDS address), so every
     // wave issues, and waits for, the same number of copies per stage.
+    constexpr int kAPerWave = (kAInst + kWaves - 1) / kWaves;
     constexpr int kBPerWave = (kBInst + kWaves - 1) / kWaves;
     constexpr int kLoadsPerStage = kAPerWave + kBPerWave;
     static_assert(BN % 64 == 0, "a B copy must stay inside one K group");
@@ -131,39 +152,61 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
+    const int group = wave / kGroupWaves;
     const int wave_m = wave % WAVES_M;
-    const int wave_n = wave / WAVES_M;
+    const int wave_n = (wave / WAVES_M) % WAVES_N;
     const int lr = lane & 15;
     const int lg = lane >> 4;
     // K split q covers stages [kt0, kt0 + nk); the host picks ksplit so none is empty
-    const int nk_all = K / kBK;
+    const int nk_all = (K + kSK - 1) / kSK;
     const int per_split = (nk_all + ksplit - 1) / ksplit;
     const int kt0 = q * per_split;
     const int nk = (nk_all - kt0) < per_split ? (nk_all - kt0) : per_split;
 
+    // K % kSK != 0: the last stage is the window [K - kSK, K) instead of one that
+    // would reach past K, so its copies need no bounds; the K it shares with the
+    // stage before is zeroed in LDS, in both operands, once it has landed
+    // (zero_tail). K < kSK: the one stage starts at 0, chunks past K copy chunk 0
+    // and are zeroed.
+    int k_last = (kt0 + nk - 1) * kSK;
+    if constexpr (kTail)
+        if (k_last >= K - kSK) k_last = K > kSK ? K - kSK : 0;
+    const bool tail = kTail && kt0 + nk == nk_all && K % kSK != 0;
+
     // ---- per-lane copy offsets (fixed), per-stage SGPR bases ----
-    // A copy j of this wave fills rows r0..r0+7 of the tile, r0 = (j * kWaves + wave) * 8.
+    // A copy a of a stage (BM / 8 per 64 K) fills 8 rows of 64 K.
+    constexpr int kAGroupInst = BM / 8;
+    auto a_copy = [&](int j) { return (j * kWaves + wave) < kAInst ? (j * kWaves + wave) : kAInst - 1; };
+    // this lane's row of A copy j, and the byte offset of its 16-byte chunk in the stage's K
+    auto a_row = [&](int j) { return (a_copy(j) % kAGroupInst) * 8 + (lane >> 3); };
+    auto a_kbyte = [&](int j) { return (a_copy(j) / kAGroupInst) * (kBK * 2) + (((lane & 7) ^ swz(a_row(j))) << 4); };
     uint32_t a_off[kAPerWave];
 #pragma unroll
     for (int j = 0; j < kAPerWave; ++j) {
-        const int row = (j * kWaves + wave) * 8 + (lane >> 3);
-        const int c = (lane & 7) ^ swz(row);
+        const int row = a_row(j);
+        const int kb = !kTail || a_kbyte(j) < 2 * K ? a_kbyte(j) : 0;
         const int lrow = (m0 + row < M ? m0 + row : M - 1) - m0;
-        a_off[j] = static_cast<uint32_t>(lrow * K * 2 + c * 16);
+        a_off[j] = static_cast<uint32_t>(lrow * K * 2 + kb);
     }
-    // B copy j covers chunks [base, base+64) of the (4 x BN) stage, base = b_copy(j) * 64.
+    // B copy j covers chunks [base, base+64) of the (4 * kGroups x BN) stage, base = b_copy(j) * 64.
     auto b_copy = [&](int j) { return (j * kWaves + wave) < kBInst ? (j * kWaves + wave) : kBInst - 1; };
     uint32_t b_off[kBPerWave];
 #pragma unroll
     for (int j = 0; j < kBPerWave; ++j) {
         const int chunk = b_copy(j) * 64 + lane;
-        const int kb = chunk / BN;
+        const int kb = !kTail || (chunk / BN) * 16 < K ? chunk / BN : 0;
         const int lcol = (n0 + chunk % BN < N ? n0 + chunk % BN : N - 1) - n0;
         b_off[j] = static_cast<uint32_t>((kb * N + lcol) * 16);
     }
-    const int64_t b_stage_bytes = static_cast<int64_t>(N) * 64;  // 4 K groups of N x 16 bytes
-    const uint8_t* a_base = reinterpret_cast<const uint8_t*>(A) + static_cast<int64_t>(m0) * K * 2 + kt0 * (kBK * 2);
-    const uint8_t* b_base = Bp + static_cast<int64_t>(n0) * 16 + kt0 * b_stage_bytes;
+    const uint8_t* a_base = reinterpret_cast<const uint8_t*>(A) + static_cast<int64_t>(m0) * K * 2;
+    const uint8_t* b_base = Bp + static_cast<int64_t>(n0) * 16;
+    // first K of stage kt; past the end (deep rings), and for a shifted last
+    // stage, that of the last stage. kInside: kt is known to lie before the last
+    auto stage_k = [&](int kt, auto inside) -> int {
+        const int k = (kt0 + kt) * kSK;
+        if constexpr (decltype(inside)::value || (!kTail && kStages == 3)) return k;
+        else return k < k_last ? k : k_last;
+    };
 
     auto stage_buf = [&](auto tag) -> uint8_t* {
         constexpr int b = decltype(tag)::value;
@@ -174,19 +217,38 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
     };
     // LDS byte address of stage buffer `tag` (a constant)
     auto stage_lds = [&](auto tag) -> uint32_t { return lds_addr_of(stage_buf(tag)); };
-    // copy i (A copies first, then B copies) of stage kt into buffer `tag`
-    auto issue_one = [&](auto tag, int kt, int i) {
+    // copy i (A copies first, then B copies) of the stage starting at K = k into
+    // buffer `tag` (16 K of the weights are N x 16 bytes)
+    auto issue_one = [&](auto tag, int k, int i) {
         const uint32_t la = stage_lds(tag);
         if (i < kAPerWave) {
-            dma16_lds(a_base + kt * (kBK * 2), a_off[i], la + ((i * kWaves + wave) * 8) * 128);
+            dma16_lds(a_base + k * 2, a_off[i], la + a_copy(i) * 1024);
         } else {
             const int j = i - kAPerWave;
-            dma16_lds(b_base + kt * b_stage_bytes, b_off[j], la + kAStage + (b_copy(j) * 64) * 16);
+            dma16_lds(b_base + static_cast<int64_t>(k) * N, b_off[j], la + kAStage + b_copy(j) * 1024);
         }
     };
-    auto issue_stage = [&](auto tag, int kt) {
+    auto issue_stage = [&](auto tag, int k) {
 #pragma unroll
-        for (int i = 0; i < kLoadsPerStage; ++i) issue_one(tag, kt, i);
+        for (int i = 0; i < kLoadsPerStage; ++i) issue_one(tag, k, i);
+    };
+    // Zeroes, in the landed last stage in buffer `tag`, the chunks this wave copied
+    // itself whose K is not the stage's own (a chunk that several waves copy is
+    // zeroed by each after its own copy has landed, so zero is the last write).
+    auto zero_tail = [&](auto tag) {
+        const int lo = K > kSK ? nk_all * kSK - K : 0, hi = K > kSK ? kSK : K;
+        const uint32_t la = stage_lds(tag);
+        using v4 = uint32_t __attribute__((ext_vector_type(4)));
+        auto clear = [&](uint32_t addr, int kk) {
+            if (kk < lo || kk >= hi)
+                *reinterpret_cast<__attribute__((address_space(3))) v4*>(static_cast<uintptr_t>(addr)) = v4{0u, 0u, 0u, 0u};
+        };
+#pragma unroll
+        for (int j = 0; j < kAPerWave; ++j) clear(la + a_copy(j) * 1024 + lane * 16, a_kbyte(j) >> 1);
+#pragma unroll
+        for (int j = 0; j < kBPerWave; ++j)
+            clear(la + kAStage + b_copy(j) * 1024 + lane * 16, ((b_copy(j) * 64 + lane) / BN) * 16);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     };
     // LDS byte offset of this lane's A operand for M repeat rm, K half kh
     auto a_lds = [&](int rm, int kh) -> int {
@@ -201,9 +263,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
         const v4 v = *reinterpret_cast<const __attribute__((address_space(3))) v4*>(static_cast<uintptr_t>(addr));
         return make_uint4(v.x, v.y, v.z, v.w);
     };
-    const uint32_t b_lane = static_cast<uint32_t>((lg * BN + wave_n * WTN + lr) * 16);
-    const uint32_t a_lane0 = static_cast<uint32_t>(a_lds(0, 0));
-    const uint32_t a_lane1 = static_cast<uint32_t>(a_lds(0, 1));
+    const uint32_t b_lane = static_cast<uint32_t>((lg * BN + wave_n * WTN + lr) * 16 + group * kBSub);
+    const uint32_t a_lane0 = static_cast<uint32_t>(a_lds(0, 0) + group * kASub);
+    const uint32_t a_lane1 = static_cast<uint32_t>(a_lds(0, 1) + group * kASub);
     auto read_b = [&](auto cur, uint4 (&braw)[RN]) {
         const uint32_t sb = stage_lds(cur) + kAStage + b_lane;
 #pragma unroll
@@ -219,6 +281,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
     using S0 = std::integral_constant<int, 0>;
     using S1 = std::integral_constant<int, 1>;
     using S2 = std::integral_constant<int, 2>;
+    using Near = std::false_type;  // stage_k: the stage may be the last one
 
     // A fragments of one K half of a stage, for every M repeat
     // (the A swizzle depends on row & 15 only, so M repeat rm adds rm * 16 rows)
@@ -347,10 +410,10 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
         // (never read) buffer, so every wait count is a constant and no
         // branch surrounds a copy; the main loop waits for those copies
         // before the epilogue reuses the buffers.
-        issue_stage(S0{}, 0);
+        issue_stage(S0{}, stage_k(0, Near{}));
         if constexpr (kStages == 3) {
             if (nk > 1) {
-                issue_stage(S1{}, 1);
+                issue_stage(S1{}, stage_k(1, Near{}));
                 wait_vmcnt<kLoadsPerStage>();
             } else {
                 wait_vmcnt<0>();
@@ -358,10 +421,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
         } else {
             static_for<kStages - 2>([&](auto i) {
                 constexpr int st = decltype(i)::value + 1;
-                issue_stage(std::integral_constant<int, st>{}, st < nk ? st : nk - 1);
+                issue_stage(std::integral_constant<int, st>{}, stage_k(st, Near{}));
             });
             wait_vmcnt<(kStages - 2) * kLoadsPerStage>();
         }
+        if constexpr (kTail)
+            if (tail && nk == 1) zero_tail(S0{});
         stage_barrier();
         read_b(S0{}, braw);
         read_a(S0{}, 0, araw[0]);
@@ -371,11 +436,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
             bqp[0] = widen_pinned(braw[0].x, braw[0].y);
             bqp[1] = widen_pinned(braw[1].x, braw[1].y);
         }
-        // kFull (three-stage ring): stages kt + 1 and kt + 2 exist (no bounds
-        // checks, so the steady-state loop body has no branches around the
-        // copies; a checked copy of the loop runs the last three to five
-        // stages). Deeper rings run every stage unchecked, the copies of
-        // stages past the end clamped to the last one.
+        // kFull (three-stage ring): stages kt + 1 and kt + 2 exist, and neither is
+        // a shifted last stage (no bounds checks, so the steady-state loop body
+        // has no branches around the copies; a checked copy of the loop runs the
+        // last three to six stages). Deeper rings run every stage unchecked,
+        // the copies of stages past the end clamped to the last one.
         auto run_stage = [&](auto cur, auto full, int kt) {
             constexpr int c = decltype(cur)::value;
             constexpr bool kFull = decltype(full)::value;
@@ -384,12 +449,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
             using Free = std::integral_constant<int, (c + kStages - 1) % kStages>;
             const bool has2 = kStages > 3 || kFull || kt + 2 < nk;
             const bool has1 = kStages > 3 || kFull || kt + 1 < nk;
-            const int kt_free = kStages > 3 && kt + kStages - 1 >= nk ? nk - 1 : kt + kStages - 1;
+            const int k_free = stage_k(kt + kStages - 1, std::bool_constant<kStages == 3 && kFull>{});
             mm_half(0, araw[0], braw, [&](int rm) {
                 if (rm == 0) read_a(cur, 1, araw[1]);
 #pragma unroll
                 for (int i = 0; i < kLoadsPerStage; ++i)
-                    if (rm == (i * RM) / kLoadsPerStage && has2) issue_one(Free{}, kt_free, i);
+                    if (rm == (i * RM) / kLoadsPerStage && has2) issue_one(Free{}, k_free, i);
             }, true);
             // mm_half widens braw before the first hook, so the hook may
             // overwrite braw with the next stage's operands
@@ -398,6 +463,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
                     // this wave's reads of stage kt have returned, stage kt + 1 has landed
                     if (has2) wait_vmcnt_lgkm0<(kStages - 2) * kLoadsPerStage>();
                     else wait_vmcnt_lgkm0<0>();
+                    if constexpr (kTail && (kStages > 3 || !kFull))
+                        if (tail && kt + 2 == nk) zero_tail(Next{});
                     stage_barrier();
                     read_b(Next{}, braw);
                     read_a(Next{}, 0, araw[0]);
@@ -408,7 +475,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
         using Tail = std::false_type;
         int kt = 0;
         if constexpr (kStages == 3) {
-            for (; kt + 5 <= nk; kt += 3) {
+            for (; kt + (tail ? 6 : 5) <= nk; kt += 3) {
                 run_stage(S0{}, Full{}, kt);
                 run_stage(S1{}, Full{}, kt + 1);
                 run_stage(S2{}, Full{}, kt + 2);
@@ -436,8 +503,10 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
             using Free = std::integral_constant<int, (c + 2) % 3>;
             if (kt + 1 < nk) wait_vmcnt<kLoadsPerStage>();
             else wait_vmcnt<0>();
+            if constexpr (kTail)
+                if (tail && kt + 1 == nk) zero_tail(cur);
             stage_barrier();
-            if (kt + 2 < nk) issue_stage(Free{}, kt + 2);
+            if (kt + 2 < nk) issue_stage(Free{}, stage_k(kt + 2, Near{}));
             uint4 braw[RN];
             read_b(cur, braw);
             uint4 araw[RM];
@@ -446,8 +515,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
             read_a(cur, 1, araw);
             mm_half(1, araw, braw, no_hook);
         };
-        issue_stage(S0{}, 0);
-        if (nk > 1) issue_stage(S1{}, 1);
+        issue_stage(S0{}, stage_k(0, Near{}));
+        if (nk > 1) issue_stage(S1{}, stage_k(1, Near{}));
         for (int kt = 0; kt < nk; kt += 3) {
             run_stage(S0{}, kt);
             if (kt + 1 < nk) run_stage(S1{}, kt + 1);
@@ -464,14 +533,44 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
     // staging writes)
     uint32_t scale_s;
     asm volatile("v_readfirstlane_b32 %0, %1" : "=s"(scale_s) : "v"(scale_raw) : "memory");
-    const float s = has_scale ? __uint_as_float(scale_s) : 1.0f;
-    // (K split: only the 32- and 64-row tiles are ever launched with ksplit > 1)
-    if constexpr (BM <= 64) if (ksplit > 1) {
+    float s = has_scale ? __uint_as_float(scale_s) : 1.0f;
+    // ---- K groups: the two groups hold partial sums of the same tile. Each keeps
+    // half of its M repeats (group 0 the first half), writes the other half to
+    // the (now free) stage buffers for the other group, and adds what that one
+    // wrote; from here on a wave's results are acc[0 .. RME), rows from erow0. ----
+    constexpr int RME = RM / kGroups;
+    const int erow0 = wave_m * WTM + group * (RME * 16);
+    if constexpr (kGroups == 2) {
+        constexpr int kPart = RME * RN * 1024;
+        static_assert(RM % 2 == 0 && kGroupWaves * kPart <= kStage, "one group's half must fit a stage buffer");
+        const int w = wave % kGroupWaves;
+        uint8_t* const mine = (group ? sbuf1 : sbuf0) + w * kPart + lane * 16;
+        const uint8_t* const theirs = (group ? sbuf0 : sbuf1) + w * kPart + lane * 16;
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's last operand reads are done
+        stage_barrier();
+#pragma unroll
+        for (int rm = 0; rm < RME; ++rm)
+#pragma unroll
+            for (int rn = 0; rn < RN; ++rn) {
+                const f32x4 give = group ? acc[rm][rn] : acc[rm + RME][rn];
+                if (group) acc[rm][rn] = acc[rm + RME][rn];
+                *reinterpret_cast<f32x4*>(mine + (rm * RN + rn) * 1024) = give;
+            }
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        stage_barrier();
+#pragma unroll
+        for (int rm = 0; rm < RME; ++rm)
+#pragma unroll
+            for (int rn = 0; rn < RN; ++rn)
+                acc[rm][rn] += *reinterpret_cast<const f32x4*>(theirs + (rm * RN + rn) * 1024);
+    }
+    // (K split: only the tiles with two K groups are ever launched with ksplit > 1)
+    if constexpr (kGroups == 2) if (ksplit > 1) {
         // ---- K split: each workgroup writes its fp32 accumulators to the
         // workspace in fragment order (lane-contiguous 16-byte pieces) and
         // bumps the tile's arrival counter; the workgroup that arrives last
-        // adds the ksplit partials in split order (deterministic), then runs
-        // the normal epilogue and re-zeroes the counter.
+        // adds the ksplit partials in split order (deterministic; its own from
+        // its registers), then runs the normal epilogue and re-zeroes the counter.
         // Ordering: the partials are only ever written and read with agent-scope
         // (sc1) accesses -- the instructions the AMDGPU memory model uses for
         // relaxed agent-scope atomic stores and loads on gfx942/gfx950 -- so
@@ -487,11 +586,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
         constexpr int kTileBytes = BM * BN * 4;
         const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
             partials + static_cast<int64_t>(lin) * ksplit * (kTileBytes / 4), 0, ksplit * kTileBytes, 0x00020000);
-        auto frag_off = [&](int rm, int rn) { return (((wave * RM + rm) * RN + rn) * 64 + lane) * 16; };
+        auto frag_off = [&](int rm, int rn) { return (((wave * RME + rm) * RN + rn) * 64 + lane) * 16; };
         constexpr int kCoherent = 16;  // sc1
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #pragma unroll
-        for (int rm = 0; rm < RM; ++rm)
+        for (int rm = 0; rm < RME; ++rm)
 #pragma unroll
             for (int rn = 0; rn < RN; ++rn)
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[rm][rn]), prs,
@@ -504,21 +603,22 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
                         static_cast<uint32_t>(ksplit - 1);
         __syncthreads();
         if (!last_flag) return;
-        // the partials are re-read in split order, kQ splits' loads in flight at a time
-        constexpr int kQ = RM * RN <= 4 ? 4 : RM * RN <= 8 ? 2 : 1;
+        // the other splits' partials are read in split order, kQ splits' loads in flight at a time
+        constexpr int kQ = RME * RN <= 4 ? 4 : 2;
+        f32x4 sum[RME][RN];
 #pragma unroll
-        for (int rm = 0; rm < RM; ++rm)
+        for (int rm = 0; rm < RME; ++rm)
 #pragma unroll
-            for (int rn = 0; rn < RN; ++rn) acc[rm][rn] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int rn = 0; rn < RN; ++rn) sum[rm][rn] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int q0 = 0; q0 < ksplit; q0 += kQ) {
-            f32x4 t[kQ][RM][RN];
+            f32x4 t[kQ][RME][RN];
 #pragma unroll
             for (int j = 0; j < kQ; ++j)
 #pragma unroll
-                for (int rm = 0; rm < RM; ++rm)
+                for (int rm = 0; rm < RME; ++rm)
 #pragma unroll
                     for (int rn = 0; rn < RN; ++rn)
-                        t[j][rm][rn] = q0 + j < ksplit
+                        t[j][rm][rn] = q0 + j < ksplit && q0 + j != q
                                            ? __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                                                                            prs, (q0 + j) * kTileBytes + frag_off(rm, rn),
                                                                            0, kCoherent))
@@ -526,27 +626,23 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
 #pragma unroll
             for (int j = 0; j < kQ; ++j)
 #pragma unroll
-                for (int rm = 0; rm < RM; ++rm)
+                for (int rm = 0; rm < RME; ++rm)
 #pragma unroll
-                    for (int rn = 0; rn < RN; ++rn) acc[rm][rn] += t[j][rm][rn];
+                    for (int rn = 0; rn < RN; ++rn) sum[rm][rn] += q0 + j == q ? acc[rm][rn] : t[j][rm][rn];
         }
+#pragma unroll
+        for (int rm = 0; rm < RME; ++rm)
+#pragma unroll
+            for (int rn = 0; rn < RN; ++rn) acc[rm][rn] = sum[rm][rn];
         if (tid == 0)  // ready for the next call on this stream
             __hip_atomic_store(&counters[lin], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 
-    if constexpr (kLora != 0) {
-        // the weight scale applies to the fp8 product only: scale first, then
-        // add the rank-R term in fp32 (one MFMA K step per 32 ranks; weights'
-        // role for U, activations' role for T, so the accumulator layout is
-        // the main loop's)
+    // ---- rank-R term T . U^T (fp32, one MFMA K step per 32 ranks; weights' role
+    // for U, activations' role for T, so the accumulator layout is the main
+    // loop's), added to dst ----
+    auto add_term = [&](f32x4 (&dst)[RM][RN], auto factors_bf16) {
         static_assert(kStage >= BM * 128 && kStage >= BN * 128, "a 64-rank chunk of T or U must fit a stage buffer");
-#pragma unroll
-        for (int rm = 0; rm < RM; ++rm)
-#pragma unroll
-            for (int rn = 0; rn < RN; ++rn)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    acc[rm][rn][i] = opaque_f32(acc[rm][rn][i] * s);
         // 64 ranks at a time, the tile's T rows and U rows are copied into the
         // (now free) stage buffers with the A operand's layout (128-byte rows,
         // chunk c at c ^ swz(row)), one round trip for the whole tile, and the
@@ -558,7 +654,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
         constexpr int kTInst = BM / 8;  // 1 KB copies: 8 rows of 64 ranks
         constexpr int kUInst = BN / 8;
         for (int r0 = 0; r0 < lora_rank; r0 += 64) {
-            const bool tail = lora_rank - r0 < 64;
+            const bool rtail = lora_rank - r0 < 64;
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of the buffers are done
             stage_barrier();                      // and every other wave's
             for (int j = wave; j < kTInst + kUInst; j += kWaves) {
@@ -566,18 +662,18 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
                 const int jj = is_t ? j : j - kTInst;
                 const int row = jj * 8 + (lane >> 3);
                 int c = (lane & 7) ^ swz(row);
-                if (tail && c >= 4) c -= 4;  // past the rank: a valid chunk, never read
+                if (rtail && c >= 4) c -= 4;  // past the rank: a valid chunk, never read
                 const int grow = is_t ? (m0 + row < M ? m0 + row : M - 1) : (n0 + row < N ? n0 + row : N - 1);
                 dma16_lds(is_t ? lora_t : lora_u, static_cast<uint32_t>((grow * lora_rank + r0 + 8 * c) * 2),
                           (is_t ? lt : lu) + jj * 1024);
             }
             wait_vmcnt<0>();
             stage_barrier();
-            for (int kh = 0; kh < (tail ? 1 : 2); ++kh) {
-                uint4 tf[RM], uf[RN];
+            for (int kh = 0; kh < (rtail ? 1 : 2); ++kh) {
+                uint4 tf[RME], uf[RN];
 #pragma unroll
-                for (int rm = 0; rm < RM; ++rm) {
-                    const int row = wave_m * WTM + rm * 16 + lr;
+                for (int rm = 0; rm < RME; ++rm) {
+                    const int row = erow0 + rm * 16 + lr;
                     tf[rm] = lds_ld16(lt + row * 128 + (((lg + 4 * kh) ^ swz(row)) << 4));
                 }
 #pragma unroll
@@ -586,19 +682,31 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
                     uf[rn] = lds_ld16(lu + row * 128 + (((lg + 4 * kh) ^ swz(row)) << 4));
                 }
 #pragma unroll
-                for (int rm = 0; rm < RM; ++rm)
+                for (int rm = 0; rm < RME; ++rm)
 #pragma unroll
                     for (int rn = 0; rn < RN; ++rn) {
-                        if constexpr (kLora == 1)
-                            acc[rm][rn] = mfma16x16x32(as_half8(uf[rn]), as_half8(tf[rm]), acc[rm][rn]);
+                        if constexpr (!decltype(factors_bf16)::value)
+                            dst[rm][rn] = mfma16x16x32(as_half8(uf[rn]), as_half8(tf[rm]), dst[rm][rn]);
                         else
-                            acc[rm][rn] = mfma16x16x32_bf16(uf[rn], tf[rm], acc[rm][rn]);
+                            dst[rm][rn] = mfma16x16x32_bf16(uf[rn], tf[rm], dst[rm][rn]);
                     }
             }
         }
+    };
+    if constexpr (kLora == 1 || kLora == 2) {
+        // the weight scale applies to the fp8 product only: scale first, then add the term
+#pragma unroll
+        for (int rm = 0; rm < RM; ++rm)
+#pragma unroll
+            for (int rn = 0; rn < RN; ++rn)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[rm][rn][i] = opaque_f32(acc[rm][rn][i] * s);
+        s = 1.0f;
+        add_term(acc, std::bool_constant<kLora == 2>{});
     }
 
-    // ---- epilogue: each wave stages its whole WTM x WTN output tile in LDS
+    // ---- epilogue: each wave stages its whole output tile (RME x RN 16 x 16 tiles) in LDS
     // (the stage buffers, free once every wave is past its last stage) with
     // one wait, then stores rows of WTN * 2 contiguous bytes ----
     const int out_col0 = n0 + wave_n * WTN;
@@ -606,7 +714,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
     constexpr int kRowBytes = WTN * 2;
     constexpr int kRowsPerStore = 64 / kCPR;     // rows one store instruction covers
     constexpr int kLanesUsed = kRowsPerStore * kCPR;
-    constexpr int kWaveBytes = WTM * kRowBytes;
+    constexpr int kWaveRows = RME * 16;
+    constexpr int kWaveBytes = kWaveRows * kRowBytes;
     constexpr int kWavesPerBuf = kStage / kWaveBytes;
     static_assert(3 * kWavesPerBuf >= kWaves, "epilogue staging must fit the stage buffers");
     const int cc = lane % kCPR;  // this lane's chunk of every row it stores
@@ -628,15 +737,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
     auto stage = [&](auto canonical) {
         constexpr bool kCanon = decltype(canonical)::value;
 #pragma unroll
-        for (int rm = 0; rm < RM; ++rm) {
+        for (int rm = 0; rm < RME; ++rm) {
             const int row = rm * 16 + lr;
 #pragma unroll
             for (int rn = 0; rn < RN; ++rn) {
                 float v[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    v[i] = kLora != 0 ? acc[rm][rn][i]
-                                      : opaque_f32(acc[rm][rn][i] * s);
+                for (int i = 0; i < 4; ++i) v[i] = kLora != 0 ? acc[rm][rn][i] : opaque_f32(acc[rm][rn][i] * s);
                 // row lr, columns 4*lg .. 4*lg+3 of this 16x16 tile: one 8-byte write
                 const int chunk = (2 * rn + (lg >> 1) + row) % kCPR;
                 uint32_t w0, w1;
@@ -659,12 +766,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
     // between the stores (vmcnt counts stores too)
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
     wave_lds_sync();                     // each wave reads only its own region
-    const int out_row0 = m0 + wave_m * WTM;
+    const int out_row0 = m0 + erow0;
 #pragma unroll
-    for (int p = 0; p < (WTM + kRowsPerStore - 1) / kRowsPerStore; ++p) {
+    for (int p = 0; p < (kWaveRows + kRowsPerStore - 1) / kRowsPerStore; ++p) {
         const int r = p * kRowsPerStore + rsub;
         const int grow = out_row0 + r;
-        if (lane < kLanesUsed && r < WTM && grow < M && gcol < N) {
+        if (lane < kLanesUsed && r < kWaveRows && grow < M && gcol < N) {
             uint4 v = *reinterpret_cast<const uint4*>(sc + r * kRowBytes + ((cc + r) % kCPR) * 16);
             if (has_bias) {
                 if constexpr (kBf16) {
@@ -688,7 +795,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void scaled_mm_lds_kernel(
     }
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int PIPE, int STAGES = 3>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int PIPE, int STAGES = 3, int GROUPS = 1, bool TAIL = false>
 bool launch_lds(const MmArgs& p, hipStream_t stream, int ksplit = 1, float* partials = nullptr,
                 uint32_t* counters = nullptr) {
     const int tiles_m = (p.M + BM - 1) / BM;
@@ -703,9 +810,9 @@ bool launch_lds(const MmArgs& p, hipStream_t stream, int ksplit = 1, float* part
     // the 100 MB intermediate written nontemporally.
     const int c_nt = p.M * p.N * 2 > (int64_t(256) << 20) ? 1 : 0;
     const dim3 grid(static_cast<uint32_t>(tiles_m * tiles_n * ksplit));
-    const dim3 block(64 * WAVES_M * WAVES_N);
+    const dim3 block(64 * WAVES_M * WAVES_N * GROUPS);
 #define FEATHER_LDS_LAUNCH_L(BF, E4, LORA)                                                                            \
-    hipLaunchKernelGGL((scaled_mm_lds_kernel<BM, BN, WAVES_M, WAVES_N, PIPE, BF, E4, LORA, STAGES>), grid, block, 0,          \
+    hipLaunchKernelGGL((scaled_mm_lds_kernel<BM, BN, WAVES_M, WAVES_N, PIPE, BF, E4, LORA, STAGES, GROUPS, TAIL>), grid, block, 0, \
                        stream, p.a, p.b, p.scale, p.bias, p.c, static_cast<int>(p.M), static_cast<int>(p.N),          \
                        static_cast<int>(p.K), p.has_scale, p.has_bias, tiles_m, tiles_n, group_m, ksplit, partials,   \
                        counters, p.lora_t, p.lora_u, static_cast<int>(p.lora_rank), c_nt)
@@ -749,7 +856,7 @@ bool launch_lds(const MmArgs& p, hipStream_t stream, int ksplit = 1, float* part
 
 template <int PIPE>
 bool launch_lds_pipe(int kernel_id, const MmArgs& p, hipStream_t stream, int ks = 1, float* partials = nullptr,
-                     uint32_t* counters = nullptr, int stages = 3) {
+                     uint32_t* counters = nullptr) {
     switch (kernel_id) {
         // 256 x 256 and 256 x 192 on 4 x 2 waves (64 x 128 / 64 x 96 wave tiles:
         // 20% fewer LDS operand bytes per stage than 2 x 4, and wide enough
@@ -760,18 +867,10 @@ bool launch_lds_pipe(int kernel_id, const MmArgs& p, hipStream_t stream, int ks 
         case kLds128x128: return launch_lds<128, 128, 2, 2, PIPE>(p, stream);
         case kLds256x192: return launch_lds<256, 192, 4, 2, PIPE>(p, stream);
         case kLds128x384: return launch_lds<128, 384, 2, 4, PIPE>(p, stream);
-        // default schedule: a five- or six-stage ring (see lds_splitk_plan)
-#define FEATHER_SK(BM_, BN_)                                                                             \
-    if constexpr (PIPE == 1) {                                                                           \
-        if (stages == 6) return launch_lds<BM_, BN_, 1, 4, PIPE, 6>(p, stream, ks, partials, counters); \
-        return launch_lds<BM_, BN_, 1, 4, PIPE, 5>(p, stream, ks, partials, counters);                  \
-    } else {                                                                                             \
-        return launch_lds<BM_, BN_, 1, 4, PIPE>(p, stream, ks, partials, counters);                     \
-    }
-        case kLdsSk64x64: FEATHER_SK(64, 64);
-        case kLdsSk64x128: FEATHER_SK(64, 128);
-        case kLdsSk32x128: FEATHER_SK(32, 128);
-#undef FEATHER_SK
+        // two K groups of 1 x 4 waves on a four- or five-stage ring of 128 K, both schedules' knob values
+        case kLdsSk64x64: return launch_lds<64, 64, 1, 4, 1, 4, 2, true>(p, stream, ks, partials, counters);
+        case kLdsSk64x128: return launch_lds<64, 128, 1, 4, 1, 4, 2, true>(p, stream, ks, partials, counters);
+        case kLdsSk32x128: return launch_lds<32, 128, 1, 4, 1, 5, 2, true>(p, stream, ks, partials, counters);
         default: return false;
     }
 }
@@ -794,37 +893,27 @@ bool launch_lds_kernel(int kernel_id, const MmArgs& p, hipStream_t stream) {
 }
 
 // Split-K plan for the 32- and 64-row tiles: as many K splits as keep the
-// grid within `target` workgroups (each split keeps at least one 64-K stage;
-// no split below 32 stages), and the stage ring's depth.
-// Measured on MI355X (weights rotated past the MALL): 64 x 64 tiles beat
-// 64 x 128 / 64 x 256 at M = 64 for N = 3072..13824, and 32 x 128 is the best
-// 32-row tile (the small-M kernel still wins at M <= 32).
-// Stage ring and grid (back to back, us, 3 / 5 / 6 stages at the grid this
-// plan picks): M=64 N=13824 K=5120 (216 tiles, one split) 31.1 / 20.9 / 20.8;
-// M=64 N=3072 K=12288 (4 splits) 22.1 / 15.9 / 15.8; M=40 N=13824 K=5120
-// 31.0 / 19.4 / 18.6; M=256 N=3072 K=3072 13.4 / 10.2 / 10.4; M=256
-// N=K=1024 5.60 / 5.18 / 5.37; M=1024 N=K=1024 6.84 / 5.69 / 5.82. The
-// three-stage ring did best with about twice the workgroups (two splits of
-// M=64 N=13824 K=5120: 24.9 us), with which the deeper rings lose (25.5):
-// one workgroup per CU with five or six stages of copies in flight streams
-// better than two sharing a CU with two each, and saves the partial-sum
-// round trip.
+// grid within `target` workgroups (each split keeps at least one stage of
+// 128 K; no split below K = 2048): each workgroup holds a CU's LDS.
+// Stage ring (back to back, us): 64 x 64 on four stages of 128 K 9.7 at M=256
+// N=K=3072, on six 9.9; 32 x 128 on five.
 SplitKPlan lds_splitk_plan(int64_t M, int64_t N, int64_t K, int target) {
     SplitKPlan pl{};
     if (M <= 0 || K % kBK != 0) return pl;
     const int bm = M <= 32 ? 32 : 64;
     const int64_t nk = K / kBK;
+    const int64_t nst = (K + 2 * kBK - 1) / (2 * kBK);  // the kernels' stages: 64 K for each of two groups
     auto splits = [&](int64_t tiles) {
         int64_t ks = target / tiles;
         // below 32 stages (K < 2048) the split's partial round trip costs more than the stages it
         // spreads (measured: M=256 N=K=1024 6.0 us unsplit vs 7.2 us in 4 splits, M=256 N=2048
         // K=512 4.7 vs 6.7 us; from K=2048 on splitting wins or ties)
         if (nk < 32) ks = 1;
-        if (ks > nk) ks = nk;
+        if (ks > nst) ks = nst;
         if (ks > 32) ks = 32;
         if (ks < 1) ks = 1;
-        const int64_t per = (nk + ks - 1) / ks;
-        ks = (nk + per - 1) / per;  // no empty split
+        const int64_t per = (nst + ks - 1) / ks;
+        ks = (nst + per - 1) / per;  // no empty split
         if (tiles > kWorkspaceCounters) ks = 1;  // more tiles than the counter region holds
         return ks;
     };
@@ -853,7 +942,6 @@ SplitKPlan lds_splitk_plan(int64_t M, int64_t N, int64_t K, int target) {
     pl.ksplit = static_cast<int>(ks);
     pl.tiles = static_cast<int>(tiles);
     pl.counter_bytes = ks > 1 ? kWorkspaceCounterBytes : 0;
-    pl.stages = nk / ks >= 64 ? 6 : 5;
     pl.workspace_bytes = ks > 1 ? pl.counter_bytes + static_cast<size_t>(tiles) * ks * bm * bn * 4 : 0;
     return pl;
 }
@@ -870,10 +958,7 @@ bool launch_lds_splitk(const MmArgs& p, void* workspace, size_t workspace_bytes,
         counters = static_cast<uint32_t*>(workspace);
         partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + pl.counter_bytes);
     }
-    const int stages = ks == pl.ksplit ? pl.stages : p.K / kBK >= 64 ? 6 : 5;
-    return lds_pipe_env() == 0 && !p.a_bf16
-               ? launch_lds_pipe<0>(pl.kernel_id, p, stream, ks, partials, counters)
-               : launch_lds_pipe<1>(pl.kernel_id, p, stream, ks, partials, counters, stages);
+    return launch_lds_pipe<1>(pl.kernel_id, p, stream, ks, partials, counters);
 }
 
 }  // namespace feather
