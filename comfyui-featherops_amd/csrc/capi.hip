@@ -91,6 +91,12 @@ int tuning_smallm_groups() {
     return g;
 }
 
+// FEATHEROPS_SPLITK, -1 when unset (see splitk_route)
+int splitk_env() {
+    const char* e = getenv("FEATHEROPS_SPLITK");
+    return e ? atoi(e) : -1;
+}
+
 // Split-K LDS tiles (64 x 64, or 32 x 128 for M <= 32) with at most 256
 // workgroups, for K % 64 == 0 and
 //   * 16 < M <= 32 and a weight larger than 4096 x 4096, unless the small-M
@@ -119,8 +125,7 @@ int tuning_smallm_groups() {
 // on every call so that tests can reach the tuple's tile kernels at small
 // shapes): 0 = never, 1 = always (K % 64 == 0).
 int splitk_route(int64_t M, int64_t N, int64_t K) {
-    const char* e = getenv("FEATHEROPS_SPLITK");
-    const int v = e ? atoi(e) : -1;
+    const int v = splitk_env();
     if (K % 64 != 0 || v == 0) return feather::kKernelNone;
     bool use = v == 1;
     if (!use && M <= 64)
@@ -152,6 +157,34 @@ int device_cus() {
         cus[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
     }
     return cus[dev];
+}
+
+// The CUs a plan fills: FEATHEROPS_SMALLM_GROUPS where it is set, else the device's.
+int plan_cus() {
+    static const bool set = getenv("FEATHEROPS_SMALLM_GROUPS") != nullptr;
+    return set ? tuning_smallm_groups() : device_cus();
+}
+
+feather::MmArgs make_args(const void* a, bool a_bf16, const uint8_t* b_prepacked, const float* scale,
+                          const uint16_t* bias, uint16_t* c, int64_t M, int64_t N, int64_t K, int has_scale,
+                          int has_bias, int b_dtype, int output_dtype) {
+    feather::MmArgs p;
+    p.a = static_cast<const uint16_t*>(a);
+    p.b = b_prepacked;
+    p.scale = scale;
+    p.bias = bias;
+    p.c = c;
+    p.M = M;
+    p.N = N;
+    p.K = K;
+    p.has_scale = has_scale ? 1 : 0;
+    p.has_bias = has_bias ? 1 : 0;
+    p.out_bf16 = output_dtype == 1;
+    p.b_e4m3 = b_dtype == FEATHER_B_E4M3FN;
+    p.a_bf16 = a_bf16;
+    p.group_m = tuning_group_m();
+    p.smallm_min_groups = tuning_smallm_groups();
+    return p;
 }
 
 int launch_status() { return hipGetLastError() == hipSuccess ? FEATHER_OK : FEATHER_ERR_LAUNCH; }
@@ -228,27 +261,67 @@ bool feather_launch_scaled_mm_ex(const void* a, int a_dtype, const uint8_t* b_pr
     if (a_dtype != FEATHER_DTYPE_F16 && a_dtype != FEATHER_DTYPE_BF16) return false;
     if (b_dtype != FEATHER_B_E4M3FN && b_dtype != FEATHER_B_E5M2) return false;
     if (output_dtype != 0 && output_dtype != 1) return false;
+    if (a_dtype == FEATHER_DTYPE_BF16 && kid != feather::kSmallM) return false;
     if (M == 0) return true;
-    feather::MmArgs p;
-    p.a = static_cast<const uint16_t*>(a);
-    p.b = b_prepacked;
-    p.scale = scale;
-    p.bias = bias;
-    p.c = c;
-    p.M = M;
-    p.N = N;
-    p.K = K;
-    p.has_scale = has_scale ? 1 : 0;
-    p.has_bias = has_bias ? 1 : 0;
-    p.out_bf16 = output_dtype == 1;
-    p.b_e4m3 = b_dtype == FEATHER_B_E4M3FN;
-    p.a_bf16 = a_dtype == FEATHER_DTYPE_BF16;
-    p.group_m = tuning_group_m();
-    p.smallm_min_groups = tuning_smallm_groups();
-    if (is_splitk(kid)) return feather::launch_lds_splitk(p, workspace, workspace_bytes, stream);
+    const feather::MmArgs p = make_args(a, a_dtype == FEATHER_DTYPE_BF16, b_prepacked, scale, bias, c, M, N, K,
+                                        has_scale, has_bias, b_dtype, output_dtype);
+    if (is_splitk(kid)) {
+        const feather::SplitKPlan pl = feather::lds_splitk_plan(M, N, K, tuning_smallm_groups());
+        const bool room = workspace != nullptr && workspace_bytes >= pl.workspace_bytes;
+        return feather::launch_tile(kid, p, room ? pl.ksplit : 1, workspace, workspace_bytes, stream);
+    }
+    // one round of 128 x 128 tiles: eight waves instead of four (the same sums in the same order)
+    if (kid == feather::kLds128x128 && feather::lds_pipe_env() != 0 &&
+        ((M + 127) / 128) * ((N + 127) / 128) <= device_cus())
+        return feather::launch_tile(feather::kMid128x128, p, 1, nullptr, 0, stream);
     if (kid == feather::kSmallM) return feather::launch_smallm_kernel(p, workspace, workspace_bytes, stream);
     if (kid >= feather::kLds256x256) return feather::launch_lds_kernel(kid, p, stream);
     return feather::launch_tile_kernel(kid, p, stream);
+}
+
+size_t feather_scaled_mm_any_m_workspace_size(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || !sizes_ok(M, N, K)) return 0;
+    if (splitk_env() >= 0) {
+        int c[5];
+        feather_scaled_mm_pick_config(M, N, K, c);
+        return feather_scaled_mm_workspace_size(M, N, K, c[0], c[1], c[2], c[3], c[4]);
+    }
+    return feather::plan_scaled_mm(M, N, K, plan_cus()).workspace_bytes;
+}
+
+int feather_scaled_mm_any_m_plan(int64_t M, int64_t N, int64_t K, int* ksplit) {
+    if (M <= 0 || !sizes_ok(M, N, K)) return feather::kKernelNone;
+    const feather::MmPlan pl = feather::plan_scaled_mm(M, N, K, plan_cus());
+    if (ksplit) *ksplit = pl.ksplit;
+    return pl.tile;
+}
+
+bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b_prepacked, const float* scale,
+                                    const uint16_t* bias, uint16_t* c, int64_t M, int64_t N, int64_t K, int has_scale,
+                                    int has_bias, int b_dtype, int output_dtype, void* workspace,
+                                    size_t workspace_bytes, hipStream_t stream) {
+    if (!sizes_ok(M, N, K)) return false;
+    if (a_dtype != FEATHER_DTYPE_F16 && a_dtype != FEATHER_DTYPE_BF16) return false;
+    if (b_dtype != FEATHER_B_E4M3FN && b_dtype != FEATHER_B_E5M2) return false;
+    if (output_dtype != 0 && output_dtype != 1) return false;
+    if (M == 0) return true;
+    if (splitk_env() >= 0) {  // forced: the tuple routes
+        int t[5];
+        feather_scaled_mm_pick_config(M, N, K, t);
+        return feather_launch_scaled_mm_ex(a, a_dtype, b_prepacked, scale, bias, c, M, N, K, has_scale, has_bias, t[0],
+                                           t[1], t[2], t[3], t[4], b_dtype, output_dtype, workspace, workspace_bytes,
+                                           stream);
+    }
+    const bool a_bf16 = a_dtype == FEATHER_DTYPE_BF16;
+    feather::MmArgs p = make_args(a, a_bf16, b_prepacked, scale, bias, c, M, N, K, has_scale, has_bias, b_dtype,
+                                  output_dtype);
+    p.smallm_min_groups = plan_cus();
+    const feather::MmPlan pl = feather::plan_scaled_mm(M, N, K, plan_cus());
+    const bool room = workspace != nullptr && workspace_bytes >= pl.workspace_bytes;
+    if (pl.tile == feather::kSmallM)
+        return feather::launch_smallm_kernel(p, pl.ksplit > 1 && room ? workspace : nullptr,
+                                             pl.ksplit > 1 && room ? workspace_bytes : 0, stream);
+    return feather::launch_tile(pl.tile, p, room ? pl.ksplit : 1, workspace, workspace_bytes, stream);
 }
 
 bool feather_launch_scaled_mm_lora(const void* a, const uint8_t* b_prepacked, const float* scale, const uint16_t* bias,
@@ -266,22 +339,8 @@ bool feather_launch_scaled_mm_lora(const void* a, const uint8_t* b_prepacked, co
     // the factor copies address T and U with 32-bit lane offsets
     if (M * rank * 2 > INT32_MAX || N * rank * 2 > INT32_MAX) return false;
     if (M == 0) return true;
-    feather::MmArgs p;
-    p.a = static_cast<const uint16_t*>(a);
-    p.b = b_prepacked;
-    p.scale = scale;
-    p.bias = bias;
-    p.c = c;
-    p.M = M;
-    p.N = N;
-    p.K = K;
-    p.has_scale = has_scale ? 1 : 0;
-    p.has_bias = has_bias ? 1 : 0;
-    p.out_bf16 = output_dtype == 1;
-    p.b_e4m3 = false;
-    p.a_bf16 = false;
-    p.group_m = tuning_group_m();
-    p.smallm_min_groups = tuning_smallm_groups();
+    feather::MmArgs p = make_args(a, false, b_prepacked, scale, bias, c, M, N, K, has_scale, has_bias, b_dtype,
+                                  output_dtype);
     p.lora_t = lora_t;
     p.lora_u = lora_u;
     p.lora_rank = rank;

@@ -49,11 +49,20 @@ enum KernelId : int {
     kLdsSk64x64 = 30,
     kLdsSk64x128 = 31,
     kLdsSk32x128 = 34,
+    // Tiles that only a plan names (feather_scaled_mm_kernel_id reports the class
+    // above that a tuple's shape falls into, never one of these)
+    kMid32x64 = 40,
+    kMid96x64 = 41,
+    kMid96x128 = 42,
+    kMid64x192 = 43,
+    kMid96x192 = 44,
+    kMid128x128 = 45,   // 2 x 4 waves, five-stage ring (kLds128x128: 2 x 2 waves, two workgroups per CU)
+    kMid128x192 = 46,
+    kTail128x256 = 47,  // 128 x 256 for K that is no multiple of 64
 };
 
 // Every launcher returns false, and launches nothing, for a variant it does not
-// have (bf16 activations are served by the split-K LDS tiles and the small-M
-// kernel with e5m2 weights only).
+// have (bf16 activations are served by the small-M kernel with e5m2 weights only).
 bool launch_tile_kernel(int kernel_id, const MmArgs& p, hipStream_t stream);
 // K-split workspace layout, shared by the small-M kernel and the split-K LDS
 // tiles: a fixed region of arrival counters (one u32 per output strip or tile)
@@ -81,7 +90,23 @@ struct SplitKPlan {
     size_t workspace_bytes; // counter region + ksplit fp32 partial tiles per output tile
 };
 SplitKPlan lds_splitk_plan(int64_t M, int64_t N, int64_t K, int target);
-// Same workspace contract as launch_smallm_kernel.
-bool launch_lds_splitk(const MmArgs& p, void* workspace, size_t workspace_bytes, hipStream_t stream);
+
+// What serves one call: a KernelId and the K split across workgroups (small-M:
+// ksplit > 1 allows that kernel's own split).
+struct MmPlan {
+    int tile = kKernelNone;
+    int ksplit = 1;
+    size_t workspace_bytes = 0;
+};
+// The variant with the least modelled time (scaled_mm_plan.hip): the same for every
+// type, so bf16 activations give the bits of their fp16 cast.
+MmPlan plan_scaled_mm(int64_t M, int64_t N, int64_t K, int cus);
+// Counter region + fp32 partial tiles of a K split (0 for ksplit 1).
+size_t tile_workspace_bytes(int tile, int64_t M, int64_t N, int ksplit);
+// Launches a tile with the given K split; ksplit > 1 needs tile_workspace_bytes() of
+// workspace (same contract as launch_smallm_kernel's).
+bool launch_tile(int tile, const MmArgs& p, int ksplit, void* workspace, size_t workspace_bytes, hipStream_t stream);
+int lds_pipe_env();  // FEATHEROPS_LDS_PIPE (1 unless set)
+bool launch_mid(int tile, const MmArgs& p, int ksplit, float* partials, uint32_t* counters, hipStream_t stream);
 
 }  // namespace feather

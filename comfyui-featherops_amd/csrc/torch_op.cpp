@@ -188,14 +188,30 @@ at::Tensor scaled_mm_any_m(const at::Tensor& a, const at::Tensor& b_prepacked, c
     TORCH_CHECK(status == FEATHER_OK, "feather_scaled_mm_pick_config failed: ", feather_status_string(status));
     const int b_dtype = b_prepacked.scalar_type() == at::kFloat8_e4m3fn ? 0 : 1;
     check_args(a, b_prepacked, scale, bias, c, cfg[0], cfg[1], cfg[2], cfg[3], cfg[4], b_dtype, false, true);
-    const Launch launch = make_launch(a, b_prepacked, scale, bias, c, cfg, b_dtype);
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(a.device().index()).stream();
+    auto launch = [&](const at::Tensor& x, int x_dtype) {
+        void* ws = nullptr;
+        size_t ws_size = 0;
+        const size_t need = feather_scaled_mm_any_m_workspace_size(M, N, K);
+        if (need) {
+            at::Tensor& t = workspace_for(a.device(), stream, need);
+            ws = t.data_ptr();
+            ws_size = static_cast<size_t>(t.numel());
+        }
+        return feather_launch_scaled_mm_any_m(
+            x.data_ptr(), x_dtype, static_cast<const uint8_t*>(b_prepacked.data_ptr()),
+            scale.has_value() ? static_cast<const float*>(scale->data_ptr()) : nullptr,
+            bias.has_value() ? static_cast<const uint16_t*>(bias->data_ptr()) : nullptr,
+            static_cast<uint16_t*>(c.data_ptr()), M, N, K, scale.has_value() ? 1 : 0, bias.has_value() ? 1 : 0,
+            b_dtype, out_dtype == at::kHalf ? 0 : 1, ws, ws_size, stream);
+    };
     bool launched;
     if (a.scalar_type() == at::kBFloat16) {
         launched = launch(a, FEATHER_DTYPE_BF16);
         if (!launched) {
             const at::Tensor a16 = at::empty(a.sizes(), a.options().dtype(at::kHalf));
             const int st = feather_bf16_to_fp16_rne(static_cast<const uint16_t*>(a.data_ptr()),
-                                                   static_cast<uint16_t*>(a16.data_ptr()), a.numel(), launch.stream);
+                                                   static_cast<uint16_t*>(a16.data_ptr()), a.numel(), stream);
             TORCH_CHECK(st == FEATHER_OK, "feather_bf16_to_fp16_rne failed: ", feather_status_string(st));
             launched = launch(a16, FEATHER_DTYPE_F16);
         }

@@ -106,6 +106,26 @@ bool feather_launch_scaled_mm_ex(const void* a, int a_dtype, const uint8_t* b_pr
                                  hipStream_t stream);
 
 /*
+ * The GEMM of feather_launch_scaled_mm_ex for a shape instead of a tuple: any M
+ * (no block divisibility; N % 16 == 0 and K % 16 == 0), the kernel, its tile and
+ * its K split chosen by a cost model of measured times. The any-M torch op calls
+ * it. With less than feather_scaled_mm_any_m_workspace_size() bytes of workspace
+ * it runs without a K split; the workspace contract is
+ * feather_launch_scaled_mm_ws's. The choice is the same for every type.
+ * bf16 activations are served by the small-M kernel with e5m2 weights; where the
+ * shape takes another kernel it returns false and launches nothing (the caller
+ * converts A and calls again). No
+ * counterpart in the reference.
+ */
+size_t feather_scaled_mm_any_m_workspace_size(int64_t M, int64_t N, int64_t K);
+/* The kernel id (csrc/scaled_mm_dispatch.h) that entry takes and, in *ksplit (may be NULL), its K split. */
+int feather_scaled_mm_any_m_plan(int64_t M, int64_t N, int64_t K, int* ksplit);
+bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b_prepacked, const float* scale,
+                                    const uint16_t* bias, uint16_t* c, int64_t M, int64_t N, int64_t K, int has_scale,
+                                    int has_bias, int b_dtype, int output_dtype, void* workspace,
+                                    size_t workspace_bytes, hipStream_t stream);
+
+/*
  * feather_launch_scaled_mm_ex without a workspace argument and without any
  * allocation. No counterpart in the reference: it is for callers that cannot
  * allocate device memory -- code under HIP graph capture, tight serving

@@ -1,0 +1,61 @@
+"""The any-M entry's planned tiles (32 x 64 up to 128 x 256, two K groups, K splits, any K): one
+shape per tile and K remainder, whole outputs against a float64 evaluation on the device, under the
+gate of gpu_util (fp32 sums in another order, two roundings to the output type)."""
+
+import ctypes
+
+import pytest
+import torch
+
+from gpu_util import assert_gemm_close_dev, lib, torch_ref_dev
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K, kernel id, K splits > 1): K a multiple of 128, of 64 only, of 16 only, below one stage
+CASES = [
+    (63, 224, 128, 40, False), (77, 128, 64, 40, False), (63, 240, 16, 40, False), (65, 256, 112, 40, False),
+    (33, 128, 2480, 40, True), (48, 128, 2304, 40, True),
+    (130, 5488, 128, 34, False), (130, 5664, 1232, 34, False), (17, 5456, 5648, 34, True),
+    (191, 5024, 432, 30, False), (333, 1712, 3904, 30, False), (33, 2864, 4464, 30, True),
+    (333, 2976, 1664, 41, False), (333, 3248, 4384, 41, False), (65, 3776, 5040, 41, True),
+    (200, 5936, 80, 31, False), (777, 2160, 2816, 31, False), (97, 4160, 3984, 31, True),
+    (333, 5504, 1264, 42, False), (333, 5408, 1728, 42, False), (200, 4640, 5520, 42, True),
+    (500, 4384, 2352, 43, False), (500, 4416, 2368, 43, False), (200, 5504, 4528, 43, True),
+    (2000, 4224, 80, 44, False), (1003, 4304, 896, 44, False), (777, 5056, 4880, 44, False),
+    (200, 6112, 16, 45, False), (1003, 1632, 128, 45, False), (777, 4064, 2704, 45, False),
+    (777, 4688, 16, 46, False), (777, 4928, 64, 46, False), (1300, 3536, 2096, 46, False),
+    (2000, 3088, 16, 47, False), (1300, 4576, 48, 47, False), (2000, 3712, 4528, 47, False),
+    (1500, 4592, 1040, 47, False),
+]
+
+
+@pytest.mark.parametrize("b_dtype,out_dtype", [(torch.float8_e5m2, torch.bfloat16), (torch.float8_e4m3fn, torch.float16)])
+@pytest.mark.parametrize("M,N,K,kid,split", CASES)
+def test_planned_tile(cuda, hk, M, N, K, kid, split, b_dtype, out_dtype):
+    ks = ctypes.c_int()
+    e4m3 = b_dtype == torch.float8_e4m3fn
+    assert lib().feather_scaled_mm_any_m_plan(M, N, K, ctypes.byref(ks)) == kid
+    assert (ks.value > 1) == split
+    print("planned tile", M, N, K, "kernel", kid, "splits", ks.value, b_dtype, flush=True)
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g, device=cuda).half()
+    w = torch.randn(N, K, generator=g, device=cuda) * 0.02
+    s = (w.abs().max() / (448.0 if e4m3 else 57344.0)).float().reshape(1)
+    bp = (w / s).to(b_dtype).view(N, K // 16, 16).permute(1, 0, 2).contiguous()
+    bias = (torch.randn(N, generator=g, device=cuda) * 0.1).to(out_dtype)
+    ref = torch_ref_dev(a, bp, s, bias, out_dtype, b_dtype=b_dtype)
+    y = hk.scaled_mm_hip_any_m(a, bp, s, bias, out_dtype)
+    assert_gemm_close_dev(y, ref, out_dtype, f"{M}x{N}x{K} kernel {kid}")
+    assert torch.equal(y.view(torch.int16), hk.scaled_mm_hip_any_m(a, bp, s, bias, out_dtype).view(torch.int16))
+    if not e4m3:  # bf16 activations: the bits of their fp16 cast (overflow, subnormals)
+        ab = a.bfloat16()
+        ab[0, :3] = torch.tensor([1.0e6, 3.0e-6, -5.0e-8], device=cuda)
+        y = hk.scaled_mm_hip_any_m(ab, bp, s, bias, out_dtype)
+        y16 = hk.scaled_mm_hip_any_m(ab.to(torch.float16), bp, s, bias, out_dtype)
+        assert torch.equal(y.view(torch.int16), y16.view(torch.int16))
+    # non-finite activations at both ends of K reach their own rows alone (the last stage's shared
+    # part and chunks past K are zeroed in both operands)
+    a[0, 0], a[M - 1, K - 1] = float("inf"), float("nan")
+    ref = torch_ref_dev(a, bp, s, None, out_dtype, b_dtype=b_dtype)
+    y = hk.scaled_mm_hip_any_m(a, bp, s, None, out_dtype)
+    assert_gemm_close_dev(y, ref, out_dtype, f"{M}x{N}x{K} kernel {kid} non-finite")

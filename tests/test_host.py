@@ -358,3 +358,41 @@ def test_lora_down_plan_leaves_no_split_empty(pkg):
             assert (ks - 1) * per < nst, (M, K, R, ks, per, nst)
             checked += 1
     assert checked > 7000
+
+
+def test_any_m_plan_is_launchable(pkg):
+    """The any-M entry's plan over random shapes of every kind it takes: a kernel that serves the
+    shape's K, no K split that would leave a workgroup without a stage, and the workspace of exactly
+    its partial tiles (256 CUs assumed without a GPU)."""
+    import ctypes
+    import random
+
+    from featherops_amd.kernel.hip import _lib
+
+    L = _lib.lib()
+    two_groups = {40: (32, 64), 34: (32, 128), 30: (64, 64), 41: (96, 64), 31: (64, 128), 42: (96, 128),
+                  43: (64, 192), 44: (96, 192)}
+    one_group = {45, 46, 47, 20, 22, 23, 24, 25, 26}
+    rng = random.Random(5)
+    seen = set()
+    for _ in range(20000):
+        M, N, K = int(2 ** rng.uniform(0, 15)), 16 * int(2 ** rng.uniform(0, 10)), 16 * int(2 ** rng.uniform(0, 10))
+        ks = ctypes.c_int(-1)
+        kid = L.feather_scaled_mm_any_m_plan(M, N, K, ctypes.byref(ks))
+        nbytes = L.feather_scaled_mm_any_m_workspace_size(M, N, K)
+        seen.add(kid)
+        if kid == 10:
+            assert M <= 64
+        elif kid in two_groups:
+            bm, bn = two_groups[kid]
+            tiles, stages = -(-M // bm) * -(-N // bn), -(-K // 128)
+            per = -(-stages // ks.value)
+            assert (ks.value - 1) * per < stages, (M, N, K, kid, ks.value)
+            assert ks.value == 1 or tiles * ks.value <= 256
+            assert nbytes == (0 if ks.value == 1 else 65536 + tiles * ks.value * bm * bn * 4)
+        else:
+            assert kid in one_group and ks.value == 1 and nbytes == 0
+            assert K % 64 == 0 or kid in (45, 46, 47), (M, N, K, kid)
+    assert seen == {10} | set(two_groups) | one_group
+    assert L.feather_scaled_mm_any_m_plan(16, 24, 64, None) == 0  # N % 16 != 0
+    assert not L.feather_launch_scaled_mm_any_m(None, 0, None, None, None, None, 16, 24, 64, 0, 0, 1, 0, None, 0, None)
