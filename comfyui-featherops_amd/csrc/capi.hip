@@ -36,8 +36,8 @@ bool known_config(int wm, int wn, int u, int rm, int rn) {
     return false;
 }
 
-// The tuple picks the output tile (BlockM x BlockN, capped at 256); the
-// LDS-DMA pipeline serves K % 64 == 0, the register-staged tile the rest.
+// The tuple picks the output tile (BlockM x BlockN, capped at 256); ids 1..6 are
+// the tiles for K % 64 != 0.
 // Shapes too small to fill the GPU with those tiles are routed first (see
 // splitk_route).
 int tile_kernel_for(int64_t M, int64_t K, int wm, int wn, int rm, int rn) {
@@ -276,7 +276,13 @@ bool feather_launch_scaled_mm_ex(const void* a, int a_dtype, const uint8_t* b_pr
         return feather::launch_tile(feather::kMid128x128, p, 1, nullptr, 0, stream);
     if (kid == feather::kSmallM) return feather::launch_smallm_kernel(p, workspace, workspace_bytes, stream);
     if (kid >= feather::kLds256x256) return feather::launch_lds_kernel(kid, p, stream);
-    return feather::launch_tile_kernel(kid, p, stream);
+    // K % 64 != 0 on the tuple's tile (256 rows: 128 x 256, which does not spill on this path)
+    switch (kid) {
+        case feather::kTile64x64: return feather::launch_tile(feather::kLdsSk64x64, p, 1, nullptr, 0, stream);
+        case feather::kTile64x128: return feather::launch_tile(feather::kLdsSk64x128, p, 1, nullptr, 0, stream);
+        case feather::kTile128x128: return feather::launch_tile(feather::kMid128x128, p, 1, nullptr, 0, stream);
+        default: return feather::launch_tile(feather::kTail128x256, p, 1, nullptr, 0, stream);
+    }
 }
 
 size_t feather_scaled_mm_any_m_workspace_size(int64_t M, int64_t N, int64_t K) {

@@ -31,6 +31,7 @@ struct MmArgs {
 // reference configs by the id they map to.
 enum KernelId : int {
     kKernelNone = 0,
+    // tuple tiles for K % 64 != 0 (served by the tiles of a plan that take any K)
     kTile256x256 = 1,
     kTile256x128 = 2,
     kTile128x256 = 3,
@@ -63,7 +64,6 @@ enum KernelId : int {
 
 // Every launcher returns false, and launches nothing, for a variant it does not
 // have (bf16 activations are served by the small-M kernel with e5m2 weights only).
-bool launch_tile_kernel(int kernel_id, const MmArgs& p, hipStream_t stream);
 // K-split workspace layout, shared by the small-M kernel and the split-K LDS
 // tiles: a fixed region of arrival counters (one u32 per output strip or tile)
 // that nothing else ever writes, then the fp32 partials. The counter region

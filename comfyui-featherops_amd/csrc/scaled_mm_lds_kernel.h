@@ -5,7 +5,7 @@
 // fp32 accumulation, scale on the accumulator, rounding to the output type,
 // bias added in the output type) for K % 64 == 0.
 //
-// Differences from the register-staged tile kernel:
+// How it works:
 //   * global -> LDS copies use gfx950's global_load_lds_dwordx4: each wave
 //     instruction moves 64 x 16 bytes straight into a contiguous 1 KB of LDS,
 //     with no VGPR staging and no ds_write. Addresses are a wave-uniform SGPR
