@@ -330,6 +330,51 @@ bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b
     return feather::launch_tile(pl.tile, p, room ? pl.ksplit : 1, workspace, workspace_bytes, stream);
 }
 
+size_t feather_scaled_mm_any_m_lora_workspace_size(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || !sizes_ok(M, N, K) || splitk_env() >= 0) return 0;
+    return feather::plan_scaled_mm_lora(M, N, K, plan_cus()).workspace_bytes;
+}
+
+bool feather_launch_scaled_mm_any_m_lora(const void* a, int a_dtype, const uint8_t* b_prepacked, const float* scale,
+                                         const uint16_t* bias, uint16_t* c, int64_t M, int64_t N, int64_t K,
+                                         int has_scale, int has_bias, const uint16_t* lora_t, const uint16_t* lora_u,
+                                         int64_t rank, int lora_dtype, int b_dtype, int output_dtype, void* workspace,
+                                         size_t workspace_bytes, hipStream_t stream) {
+    if (!sizes_ok(M, N, K) || M == 0) return false;
+    if (a_dtype != FEATHER_DTYPE_F16 && a_dtype != FEATHER_DTYPE_BF16) return false;
+    if (b_dtype != FEATHER_B_E5M2 || (output_dtype != 0 && output_dtype != 1)) return false;
+    if (lora_dtype != FEATHER_DTYPE_F16 && lora_dtype != FEATHER_DTYPE_BF16) return false;
+    if (lora_t == nullptr || lora_u == nullptr || rank <= 0 || rank % 32 != 0) return false;
+    if ((reinterpret_cast<uintptr_t>(lora_t) | reinterpret_cast<uintptr_t>(lora_u)) % 16 != 0) return false;
+    // the factor copies address T and U with 32-bit lane offsets
+    if (rank > INT32_MAX / 2 || M * rank * 2 > INT32_MAX || N * rank * 2 > INT32_MAX) return false;
+    feather::MmArgs p = make_args(a, a_dtype == FEATHER_DTYPE_BF16, b_prepacked, scale, bias, c, M, N, K, has_scale,
+                                  has_bias, b_dtype, output_dtype);
+    p.smallm_min_groups = plan_cus();
+    p.lora_t = lora_t;
+    p.lora_u = lora_u;
+    p.lora_rank = rank;
+    p.lora_dtype = lora_dtype == FEATHER_DTYPE_F16 ? 1 : 2;
+    // Where the term is rounded goes by the tuple route's kernel id, whatever tile the
+    // plan takes: ids 20..29 add it to the fp32 accumulator, the others in the output type.
+    int t[5];
+    feather_scaled_mm_pick_config(M, N, K, t);
+    const int kid = feather_scaled_mm_kernel_id(M, N, K, t[0], t[1], t[2], t[3], t[4]);
+    p.lora_after = kid < feather::kLds256x256 || is_splitk(kid);
+    if (splitk_env() >= 0)  // forced: the tuple routes
+        return !p.lora_after &&
+               feather::launch_tile(kid == feather::kLds128x384 ? static_cast<int>(feather::kLds256x192) : kid, p, 1,
+                                    nullptr, 0, stream);
+    const feather::MmPlan pl = feather::plan_scaled_mm_lora(M, N, K, plan_cus());
+    const bool room = workspace != nullptr && workspace_bytes >= pl.workspace_bytes;
+    if (pl.tile == feather::kSmallM) return p.lora_after && feather::launch_smallm_kernel(p, nullptr, 0, stream);
+    const bool large = pl.tile >= feather::kLds256x256 && pl.tile < feather::kLdsSk64x64;
+    if (large && p.lora_after) return false;
+    // the 128 x 384 tile's stage buffers cannot hold 64 ranks of its U rows
+    return feather::launch_tile(pl.tile == feather::kLds128x384 ? static_cast<int>(feather::kLds256x192) : pl.tile, p,
+                                room ? pl.ksplit : 1, workspace, workspace_bytes, stream);
+}
+
 bool feather_launch_scaled_mm_lora(const void* a, const uint8_t* b_prepacked, const float* scale, const uint16_t* bias,
                                    uint16_t* c, int64_t M, int64_t N, int64_t K, int has_scale, int has_bias,
                                    const uint16_t* lora_t, const uint16_t* lora_u, int64_t rank, int lora_dtype,

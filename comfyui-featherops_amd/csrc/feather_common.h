@@ -79,6 +79,20 @@ __device__ __forceinline__ uint32_t f32x2_to_out_bits(float a, float b) {
     // the M=32768 N=13824 K=5120 epilogue
     else return static_cast<uint32_t>(f32_to_half_bits(a)) | (static_cast<uint32_t>(f32_to_half_bits(b)) << 16);
 }
+// Two fp32 -> bf16 (via_bf16) or fp16, and those to the output type, packed: the
+// roundings of a product held in one 16-bit type and converted to another.
+template <bool kBf16>
+__device__ __forceinline__ uint32_t round_via(float a, float b, bool via_bf16) {
+    if (via_bf16) {
+        const uint32_t r = f32x2_to_bf16x2_bits(a, b);
+        if constexpr (kBf16) return r;
+        return f32x2_to_out_bits<false>(bits_f32(r << 16), bits_f32(r & 0xffff0000u));
+    }
+    const uint32_t h = f32x2_to_out_bits<false>(a, b);
+    if constexpr (!kBf16) return h;
+    return f32x2_to_bf16x2_bits(half_bits_to_f32(static_cast<uint16_t>(h & 0xffffu)),
+                                half_bits_to_f32(static_cast<uint16_t>(h >> 16)));
+}
 template <bool kBf16>
 __device__ __forceinline__ float out_bits_to_f32(uint16_t b) {
     if constexpr (kBf16) return bf16_bits_to_f32(b);

@@ -20,11 +20,12 @@ struct MmArgs {
     bool a_bf16;             // activations are bf16 (converted to fp16 in the kernel; e5m2 weights only)
     int group_m;             // tile raster group height (0 = default)
     int smallm_min_groups;   // small-M: workgroup count the K split aims for (0 = default)
-    // rank-R epilogue update C += T . U^T (LDS tiles only): T (M, R), U (N, R)
+    // rank-R term C += T . U^T: T (M, R), U (N, R)
     const uint16_t* lora_t = nullptr;
     const uint16_t* lora_u = nullptr;
     int64_t lora_rank = 0;
     int lora_dtype = 0;      // 0 none, 1 fp16 factors, 2 bf16 factors
+    bool lora_after = false; // added to the finished result, in the output type
 };
 
 // Kernel variants. Values are stable: the Python autotuner de-duplicates
@@ -101,6 +102,9 @@ struct MmPlan {
 // The variant with the least modelled time (scaled_mm_plan.hip): the same for every
 // type, so bf16 activations give the bits of their fp16 cast.
 MmPlan plan_scaled_mm(int64_t M, int64_t N, int64_t K, int cus);
+// The same for a call with a rank-R term: the small-M kernel only where its lean form, which adds it, serves the shape.
+MmPlan plan_scaled_mm_lora(int64_t M, int64_t N, int64_t K, int cus);
+bool smallm_is_lean(int64_t M, int64_t N, int64_t K, int target_groups, bool allow_split);
 // Counter region + fp32 partial tiles of a K split (0 for ksplit 1).
 size_t tile_workspace_bytes(int tile, int64_t M, int64_t N, int ksplit);
 // Launches a tile with the given K split; ksplit > 1 needs tile_workspace_bytes() of

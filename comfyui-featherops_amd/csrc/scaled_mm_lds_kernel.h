@@ -78,7 +78,10 @@ constexpr int kBK = 64;
 
 
 // kLora: 0 = none, 1 = fp16 factors, 2 = bf16 factors (T is M x R, U is N x R,
-// both row-major with R % 32 == 0 and 16-byte aligned rows)
+// both row-major with R % 32 == 0 and 16-byte aligned rows), 3 = either, by
+// lora_flags: bit 0 = bf16 factors, bit 1 = the term is rounded to the factors'
+// type and to the output type and added to the finished result in the output
+// type (a separate pass's arithmetic) instead of joining the fp32 accumulator
 // kGroups: 1, or 2 = two groups of WAVES_M x WAVES_N waves share a stage of 2 x
 // 64 K, each multiplying its own 64 of it for the whole tile (see the K groups
 // paragraph in the file header). kTail: K need not be a multiple of the stage
@@ -88,7 +91,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
     const uint16_t* __restrict__ A, const uint8_t* __restrict__ Bp, const float* __restrict__ scale,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M, int N, int K, int has_scale, int has_bias,
     int tiles_m, int tiles_n, int group_m, int ksplit, float* __restrict__ partials, uint32_t* __restrict__ counters,
-    const uint16_t* __restrict__ lora_t, const uint16_t* __restrict__ lora_u, int lora_rank, int c_nontemporal) {
+    const uint16_t* __restrict__ lora_t, const uint16_t* __restrict__ lora_u, int lora_rank, int lora_flags,
+    int c_nontemporal) {
     constexpr int kGroupWaves = WAVES_M * WAVES_N;
     constexpr int kWaves = kGroupWaves * kGroups;
     constexpr int WTM = BM / WAVES_M;
@@ -706,6 +710,28 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
         s = 1.0f;
         add_term(acc, std::bool_constant<kLora == 2>{});
     }
+    [[maybe_unused]] f32x4 term[kLora == 3 ? RM : 1][RN];
+    [[maybe_unused]] const bool term_bf16 = (lora_flags & 1) != 0, term_after = (lora_flags & 2) != 0;
+    if constexpr (kLora == 3) {
+#pragma unroll
+        for (int rm = 0; rm < RM; ++rm)
+#pragma unroll
+            for (int rn = 0; rn < RN; ++rn) term[rm][rn] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (term_after) {
+            if (term_bf16) add_term(term, std::true_type{});
+            else add_term(term, std::false_type{});
+        } else {
+#pragma unroll
+            for (int rm = 0; rm < RME; ++rm)
+#pragma unroll
+                for (int rn = 0; rn < RN; ++rn)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[rm][rn][i] = opaque_f32(acc[rm][rn][i] * s);
+            s = 1.0f;
+            if (term_bf16) add_term(acc, std::true_type{});
+            else add_term(acc, std::false_type{});
+        }
+    }
 
     // ---- epilogue: each wave stages its whole output tile (RME x RN 16 x 16 tiles) in LDS
     // (the stage buffers, free once every wave is past its last stage) with
@@ -727,8 +753,29 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
     const uint4 b8 = has_bias && lane < kLanesUsed && gcol < N ? load_bias8(bias + gcol) : make_uint4(0u, 0u, 0u, 0u);
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's last operand reads are done
     stage_barrier();
-    uint8_t* sc = (wave / kWavesPerBuf == 0 ? sbuf0 : wave / kWavesPerBuf == 1 ? sbuf1 : sbuf2) +
-                  (wave % kWavesPerBuf) * kWaveBytes;
+    auto staging = [&](int buf) -> uint8_t* {
+        uint8_t* const b = buf == 0 ? sbuf0 : buf == 1 ? sbuf1 : buf == 2 ? sbuf2 : sbufx + (buf - 3) * kStage;
+        return b + (wave % kWavesPerBuf) * kWaveBytes;
+    };
+    uint8_t* sc = staging(wave / kWavesPerBuf);
+    // a separately added term is staged like the result, in the buffers behind it
+    constexpr int kResultBufs = (kWaves + kWavesPerBuf - 1) / kWavesPerBuf;
+    static_assert(kLora != 3 || 2 * kResultBufs <= kStages, "result and term must fit the stage buffers");
+    [[maybe_unused]] uint8_t* const st_term = staging(wave / kWavesPerBuf + (kLora == 3 ? kResultBufs : 0));
+    if constexpr (kLora == 3) {
+        if (term_after) {
+#pragma unroll
+            for (int rm = 0; rm < RME; ++rm)
+#pragma unroll
+                for (int rn = 0; rn < RN; ++rn) {
+                    const int row = rm * 16 + lr;
+                    const int chunk = (2 * rn + (lg >> 1) + row) % kCPR;
+                    const f32x4 v = term[rm][rn];
+                    *reinterpret_cast<uint2*>(st_term + row * kRowBytes + chunk * 16 + (lg & 1) * 8) =
+                        make_uint2(round_via<kBf16>(v[0], v[1], term_bf16), round_via<kBf16>(v[2], v[3], term_bf16));
+                }
+        }
+    }
     // chunk c of staged row r sits at (c + r) % kCPR (spreads the rows of one
     // write over the LDS banks). bf16 outputs are converted without NaN
     // canonicalisation first; a wave that produced a NaN stages again with
@@ -744,7 +791,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
             for (int rn = 0; rn < RN; ++rn) {
                 float v[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = kLora != 0 ? acc[rm][rn][i] : opaque_f32(acc[rm][rn][i] * s);
+                for (int i = 0; i < 4; ++i)
+                    v[i] = kLora == 1 || kLora == 2 ? acc[rm][rn][i] : opaque_f32(acc[rm][rn][i] * s);
                 // row lr, columns 4*lg .. 4*lg+3 of this 16x16 tile: one 8-byte write
                 const int chunk = (2 * rn + (lg >> 1) + row) % kCPR;
                 uint32_t w0, w1;
@@ -785,6 +833,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
                     add_bias8<false>(v, b8);
                 }
             }
+            if constexpr (kLora == 3)
+                if (term_after)
+                    add_bias8<kBf16>(v, *reinterpret_cast<const uint4*>(st_term + r * kRowBytes + ((cc + r) % kCPR) * 16));
             uint4* dst = reinterpret_cast<uint4*>(C + static_cast<int64_t>(grow) * N + gcol);
             if (c_nontemporal) {
                 typedef uint32_t u32x4_nt __attribute__((ext_vector_type(4)));
@@ -794,6 +845,14 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
             }
         }
     }
+}
+
+// Whether the epilogue can stage a separately added term beside the result (see
+// kResultBufs) and hold 64 ranks of T and U in a stage buffer each.
+template <int BM, int BN, int WAVES, int GROUPS, int STAGES>
+constexpr bool term_fits() {
+    constexpr int kStage = GROUPS * (BM * 128 + BN * 64), kPerBuf = kStage / (BM * BN * 2 / WAVES);
+    return 2 * ((WAVES + kPerBuf - 1) / kPerBuf) <= STAGES && kStage >= BM * 128 && kStage >= BN * 128;
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int PIPE, int STAGES = 3, int GROUPS = 1, bool TAIL = false>
@@ -816,13 +875,22 @@ bool launch_lds(const MmArgs& p, hipStream_t stream, int ksplit = 1, float* part
     hipLaunchKernelGGL((scaled_mm_lds_kernel<BM, BN, WAVES_M, WAVES_N, PIPE, BF, E4, LORA, STAGES, GROUPS, TAIL>),     \
                        grid, block, 0, stream, p.a, p.b, p.scale, p.bias, p.c, static_cast<int>(p.M),                 \
                        static_cast<int>(p.N), static_cast<int>(p.K), p.has_scale, p.has_bias, tiles_m, tiles_n,       \
-                       group_m, ksplit, partials, counters, p.lora_t, p.lora_u, static_cast<int>(p.lora_rank), c_nt)
+                       group_m, ksplit, partials, counters, p.lora_t, p.lora_u, static_cast<int>(p.lora_rank),         \
+                       (p.lora_dtype == 2 ? 1 : 0) | (p.lora_after ? 2 : 0), c_nt)
 #define FEATHER_LDS_LAUNCH(BF, E4) FEATHER_LDS_LAUNCH_L(BF, E4, 0)
     if (p.lora_dtype != 0) {
+        // rank-R epilogue with the factors' type and the place of the rounding as
+        // arguments: the planned tiles (fp16 activations, e5m2 weights, with or without a K split)
+        if constexpr (TAIL && term_fits<BM, BN, WAVES_M * WAVES_N * GROUPS, GROUPS, STAGES>()) {
+            if (p.a_bf16 || p.b_e4m3) return false;
+            if (p.out_bf16) FEATHER_LDS_LAUNCH_L(true, false, 3);
+            else FEATHER_LDS_LAUNCH_L(false, false, 3);
+            return true;
+        }
         // rank-R epilogue: the default schedule's large tiles, fp16 activations,
         // e5m2 weights, no K split
         // (the T and U chunks must fit a stage buffer: not the 128 x 384 tile)
-        if constexpr (PIPE == 1 && BM >= 128 && BM * 128 + BN * 64 >= (BM > BN ? BM : BN) * 128) {
+        if constexpr (PIPE == 1 && !TAIL && BM >= 128 && BM * 128 + BN * 64 >= (BM > BN ? BM : BN) * 128) {
             if (p.a_bf16 || p.b_e4m3 || ksplit != 1) return false;
             if (p.lora_dtype == 1) {
                 if (p.out_bf16) FEATHER_LDS_LAUNCH_L(true, false, 1);

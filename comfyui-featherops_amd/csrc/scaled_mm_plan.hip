@@ -85,9 +85,10 @@ const TileCost* tile_cost(int tile) {
     return nullptr;
 }
 
-MmPlan make_plan(int64_t M, int64_t N, int64_t K, int cus) {
+MmPlan make_plan(int64_t M, int64_t N, int64_t K, int cus, bool lora) {
     MmPlan best;
-    if (M <= 16) {
+    const bool lean = M <= 32 && smallm_is_lean(M, N, K, cus, M <= 16);
+    if (M <= 16 && (!lora || lean)) {
         // one row tile: the small-M kernel and its own plan. The 32 x 64 tile took up to 13%
         // less on 11 of 70 shapes, all with wide weights (M=16 N=13824 K=5120 13.2 vs 14.3
         // us, M=1 N=12288 K=3072 8.7 vs 10.0), but bf16 activations would need a cast pass
@@ -124,7 +125,7 @@ MmPlan make_plan(int64_t M, int64_t N, int64_t K, int cus) {
         }
     }
     best.workspace_bytes = tile_workspace_bytes(best.tile, M, N, best.ksplit);
-    if (M <= 48) {
+    if (M > 16 && M <= 48 && (!lora || lean)) {
         // bf16 activations cost a cast pass (3.5 us and more) before a tile, none on the
         // small-M kernel, and both types take one plan: where a weight is too small to
         // make the tiles the better choice for most rows, they have to win by that much
@@ -146,24 +147,23 @@ size_t tile_workspace_bytes(int tile, int64_t M, int64_t N, int ksplit) {
 
 // The plan is a pure function of its arguments and costs about a microsecond, so each
 // thread keeps the last few.
-MmPlan plan_scaled_mm(int64_t M, int64_t N, int64_t K, int cus) {
+static MmPlan plan(int64_t M, int64_t N, int64_t K, int cus, bool lora) {
     struct Entry {
         int64_t M = -1, N = 0, K = 0;
         int cus = 0;
+        bool lora = false;
         MmPlan plan;
     };
     static thread_local Entry memo[64];
     const uint64_t h = static_cast<uint64_t>(M) * 0x9e3779b97f4a7c15ull + static_cast<uint64_t>(N) * 0xc2b2ae3d27d4eb4full +
-                       static_cast<uint64_t>(K) * 0x165667b19e3779f9ull;
-    Entry& e = memo[h >> 58];
-    if (e.M != M || e.N != N || e.K != K || e.cus != cus) {
-        e.plan = make_plan(M, N, K, cus);
-        e.M = M;
-        e.N = N;
-        e.K = K;
-        e.cus = cus;
-    }
+                       static_cast<uint64_t>(K) * 0x165667b19e3779f9ull + (lora ? 1u : 0u);
+    Entry& e = memo[(h ^ (h >> 29)) * 0xbf58476d1ce4e5b9ull >> 58];
+    if (e.M != M || e.N != N || e.K != K || e.cus != cus || e.lora != lora)
+        e = Entry{M, N, K, cus, lora, make_plan(M, N, K, cus, lora)};
     return e.plan;
 }
+
+MmPlan plan_scaled_mm(int64_t M, int64_t N, int64_t K, int cus) { return plan(M, N, K, cus, false); }
+MmPlan plan_scaled_mm_lora(int64_t M, int64_t N, int64_t K, int cus) { return plan(M, N, K, cus, true); }
 
 }  // namespace feather

@@ -257,13 +257,20 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_smallm_kernel(
 //     measured ~0.4 us slower at M=16, K=N=4096).
 // M=16, K=N=4096, 24 rotated weights, back-to-back launches: 5.87 us against
 // 6.45 us for the general kernel on the same box.
-template <int MT, bool kBf16, bool kE4m3, bool kABf16>
+// kLora: adds the rank-R term T . U^T (T (M, R), U (N, R), fp16 or bf16 by lora_bf16,
+// R % 32 == 0) to the finished result in the output type: wave t multiplies row tile
+// t's 16 x 16 product (fp32 MFMA sums, rounded to the factors' type and to the output
+// type) after its share of the stream, while the other waves write their sums.
+template <int MT, bool kBf16, bool kE4m3, bool kABf16, bool kLora>
 __global__ __launch_bounds__(64 * kWaves) void scaled_mm_m16_kernel(const uint16_t* __restrict__ A,
                                                                      const uint8_t* __restrict__ Bp,
                                                                      const float* __restrict__ scale,
                                                                      const uint16_t* __restrict__ bias,
                                                                      uint16_t* __restrict__ C, int M, int N, int K,
-                                                                     int has_scale, int has_bias) {
+                                                                     int has_scale, int has_bias,
+                                                                     const uint16_t* __restrict__ lora_t,
+                                                                     const uint16_t* __restrict__ lora_u,
+                                                                     int lora_rank, int lora_bf16) {
     constexpr int U = 4 / MT;  // stages in flight per wave (the slabs fill 128 KB of LDS)
     constexpr int kStageSlab = MT * kSlabTile;
     constexpr int kRedStride = 17;
@@ -274,6 +281,7 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_m16_kernel(const uint16
     // row tiles overlay it on the slabs (there is no room beside them)
     constexpr bool kOwnRed = MT == 1;
     __shared__ __attribute__((aligned(16))) float red_own[kOwnRed ? kWaves * 16 * MT * kRedStride : 1];
+    __shared__ __attribute__((aligned(16))) uint16_t term[kLora ? MT * 16 * 16 : 1];  // the rank-R term in the output type, [row][column]
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
@@ -384,6 +392,22 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_m16_kernel(const uint16
     for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) red[(wave * 16 * MT + t * 16 + lr) * kRedStride + 4 * lg + i] = acc[t][i];
+    if constexpr (kLora) {
+        if (wave < MT) {
+            const int row = wave * 16 + lr;
+            const uint16_t* tp = lora_t + static_cast<int64_t>(row < M ? row : M - 1) * lora_rank + lg * 8;
+            const uint16_t* up = lora_u + static_cast<int64_t>(n0 + lr) * lora_rank + lg * 8;
+            f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int r = 0; r < lora_rank; r += 32) {
+                const uint4 tf = *reinterpret_cast<const uint4*>(tp + r);
+                const uint4 uf = *reinterpret_cast<const uint4*>(up + r);
+                if (lora_bf16) sum = mfma16x16x32_bf16(uf, tf, sum);
+                else sum = mfma16x16x32(as_half8(uf), as_half8(tf), sum);
+            }
+            *reinterpret_cast<uint2*>(&term[row * 16 + 4 * lg]) = make_uint2(
+                round_via<kBf16>(sum[0], sum[1], lora_bf16 != 0), round_via<kBf16>(sum[2], sum[3], lora_bf16 != 0));
+        }
+    }
     __syncthreads();
     if (tid < 256 * MT) {
         const int r = tid >> 4;
@@ -395,6 +419,8 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_m16_kernel(const uint16
         if (r < M) {
             uint16_t o = f32_to_out_bits<kBf16>(opaque_f32(sum * s));
             if (has_bias) o = f32_to_out_bits<kBf16>(out_bits_to_f32<kBf16>(o) + out_bits_to_f32<kBf16>(b));
+            if constexpr (kLora)
+                o = f32_to_out_bits<kBf16>(out_bits_to_f32<kBf16>(o) + out_bits_to_f32<kBf16>(term[r * 16 + c]));
             C[static_cast<int64_t>(r) * N + n0 + c] = o;
         }
     }
@@ -404,10 +430,23 @@ template <int MT>
 bool launch_m16(const MmArgs& p, hipStream_t stream) {
     const dim3 grid(static_cast<uint32_t>(p.N / 16));
     const dim3 block(64 * kWaves);
-#define FEATHER_M16_LAUNCH(BF, E4, AB)                                                                             \
-    hipLaunchKernelGGL((scaled_mm_m16_kernel<MT, BF, E4, AB>), grid, block, 0, stream, p.a, p.b, p.scale, p.bias, \
-                       p.c, static_cast<int>(p.M), static_cast<int>(p.N), static_cast<int>(p.K), p.has_scale,       \
-                       p.has_bias)
+#define FEATHER_M16_LAUNCH_L(BF, E4, AB, LORA)                                                                   \
+    hipLaunchKernelGGL((scaled_mm_m16_kernel<MT, BF, E4, AB, LORA>), grid, block, 0, stream, p.a, p.b, p.scale,     \
+                       p.bias, p.c, static_cast<int>(p.M), static_cast<int>(p.N), static_cast<int>(p.K),            \
+                       p.has_scale, p.has_bias, p.lora_t, p.lora_u, static_cast<int>(p.lora_rank),                  \
+                       p.lora_dtype == 2 ? 1 : 0)
+#define FEATHER_M16_LAUNCH(BF, E4, AB) FEATHER_M16_LAUNCH_L(BF, E4, AB, false)
+    if (p.lora_dtype != 0) {
+        if (p.b_e4m3 || !p.lora_after) return false;
+        if (p.a_bf16) {
+            if (p.out_bf16) FEATHER_M16_LAUNCH_L(true, false, true, true);
+            else FEATHER_M16_LAUNCH_L(false, false, true, true);
+        } else {
+            if (p.out_bf16) FEATHER_M16_LAUNCH_L(true, false, false, true);
+            else FEATHER_M16_LAUNCH_L(false, false, false, true);
+        }
+        return true;
+    }
     if (p.a_bf16) {
         if (p.b_e4m3) return false;  // bf16 activations: e5m2 weights only, as on the other small-M routes
         if (p.out_bf16) FEATHER_M16_LAUNCH(true, false, true);
@@ -422,6 +461,7 @@ bool launch_m16(const MmArgs& p, hipStream_t stream) {
         else FEATHER_M16_LAUNCH(false, false, false);
     }
 #undef FEATHER_M16_LAUNCH
+#undef FEATHER_M16_LAUNCH_L
     return true;
 }
 
@@ -565,6 +605,12 @@ static bool m16_disabled() {
     return off;
 }
 
+bool smallm_is_lean(int64_t M, int64_t N, int64_t K, int target_groups, bool allow_split) {
+    if (M <= 0 || M > 32) return false;
+    const SmallmPlan pl = smallm_plan(M, N, K, target_groups, allow_split);
+    return pl.ks == 1 && pl.ct == 1 && M * K * 2 < (int64_t(1) << 32) && K % 64 == 0 && N % 16 == 0 && !m16_disabled();
+}
+
 bool launch_smallm_kernel(const MmArgs& p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     if (p.M <= 0 || p.M > 64) return false;
     const int mt = mt_of(p.M);
@@ -586,6 +632,7 @@ bool launch_smallm_kernel(const MmArgs& p, void* workspace, size_t workspace_byt
     const bool lds_a = p.M * p.K * 2 < (int64_t(1) << 32);
     if (mt <= 2 && ks == 1 && !wide && lds_a && p.K % 64 == 0 && p.N % 16 == 0 && !m16_disabled())
         return mt == 1 ? launch_m16<1>(p, stream) : launch_m16<2>(p, stream);
+    if (p.lora_dtype != 0) return false;  // only the lean kernel adds a rank-R term
     switch (mt) {
         case 1:
             if (lds_a) return wide ? launch_mt<1, 4, true>(p, ks, partials, counters, stream)

@@ -246,9 +246,10 @@ at::Tensor scaled_mm_configured_meta(const at::Tensor& a, const at::Tensor& b_pr
 // feather_ops::scaled_mm_any_m_lora: scaled_mm_any_m plus the unmerged-LoRA
 // term T . U^T (reference comfy_feather/lora.py:4-35, after F.linear(x, A);
 // the strengths are folded into T by the caller). T (M, R) and U (N, R) are
-// contiguous fp16 or bf16 with R % 32 == 0. On the large LDS tiles the term is
-// added to the scaled fp32 accumulator before rounding; on every other route
-// the GEMM runs as scaled_mm_any_m and the term is added to C afterwards.
+// contiguous fp16 or bf16 with R % 32 == 0. The GEMM's epilogue adds the term: to the
+// scaled fp32 accumulator where the tuple route takes a large LDS tile, else to the
+// finished result in the output type. Where no kernel does (e4m3fn weights, K % 64 != 0
+// on wide grids) the GEMM runs as scaled_mm_any_m and a second pass adds the term to C.
 at::Tensor scaled_mm_any_m_lora(const at::Tensor& a, const at::Tensor& b_prepacked,
                                 const std::optional<at::Tensor>& scale, const std::optional<at::Tensor>& bias,
                                 at::ScalarType out_dtype, const at::Tensor& lora_t, const at::Tensor& lora_u) {
@@ -275,37 +276,37 @@ at::Tensor scaled_mm_any_m_lora(const at::Tensor& a, const at::Tensor& b_prepack
     const int status = feather_scaled_mm_pick_config(M, N, K, cfg);
     TORCH_CHECK(status == FEATHER_OK, "feather_scaled_mm_pick_config failed: ", feather_status_string(status));
     const int b_dtype = b_prepacked.scalar_type() == at::kFloat8_e4m3fn ? 0 : 1;
-    int kid = feather_scaled_mm_kernel_id(M, N, K, cfg[0], cfg[1], cfg[2], cfg[3], cfg[4]);
-    if (kid == 26) {
-        // the 128 x 384 tile's stage buffers cannot hold 64 ranks of its U rows, so it has no rank-R
-        // epilogue: the 256 x 192 tile covers the same grids (256 tiles at M = 4096, N = 3072)
-        const int alt[5] = {2, 4, 4, 8, 3};
-        for (int i = 0; i < 5; ++i) cfg[i] = alt[i];
-        kid = feather_scaled_mm_kernel_id(M, N, K, cfg[0], cfg[1], cfg[2], cfg[3], cfg[4]);
-    }
-    // the fused epilogue: large LDS tiles (kernel ids 20-29 but 26), e5m2 weights
-    if (kid >= 20 && kid < 30 && b_dtype == 1) {
-        at::Tensor c = at::empty({M, N}, a.options().dtype(out_dtype));
-        check_args(a, b_prepacked, scale, bias, c, cfg[0], cfg[1], cfg[2], cfg[3], cfg[4], b_dtype, false, true);
-        const hipStream_t stream = c10::hip::getCurrentHIPStream(a.device().index()).stream();
-        at::Tensor a16 = a;
-        if (a.scalar_type() == at::kBFloat16) {  // the large tiles take fp16 activations
-            a16 = at::empty(a.sizes(), a.options().dtype(at::kHalf));
-            const int st = feather_bf16_to_fp16_rne(static_cast<const uint16_t*>(a.data_ptr()),
-                                                    static_cast<uint16_t*>(a16.data_ptr()), a.numel(), stream);
-            TORCH_CHECK(st == FEATHER_OK, "feather_bf16_to_fp16_rne failed: ", feather_status_string(st));
+    at::Tensor c = at::empty({M, N}, a.options().dtype(out_dtype));
+    check_args(a, b_prepacked, scale, bias, c, cfg[0], cfg[1], cfg[2], cfg[3], cfg[4], b_dtype, false, true);
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(a.device().index()).stream();
+    auto launch = [&](const at::Tensor& x, int x_dtype) {
+        void* ws = nullptr;
+        size_t ws_size = 0;
+        const size_t need = feather_scaled_mm_any_m_lora_workspace_size(M, N, K);
+        if (need) {
+            at::Tensor& t = workspace_for(a.device(), stream, need);
+            ws = t.data_ptr();
+            ws_size = static_cast<size_t>(t.numel());
         }
-        const bool launched = feather_launch_scaled_mm_lora(
-            a16.data_ptr(), static_cast<const uint8_t*>(b_prepacked.data_ptr()),
+        return feather_launch_scaled_mm_any_m_lora(
+            x.data_ptr(), x_dtype, static_cast<const uint8_t*>(b_prepacked.data_ptr()),
             scale.has_value() ? static_cast<const float*>(scale->data_ptr()) : nullptr,
             bias.has_value() ? static_cast<const uint16_t*>(bias->data_ptr()) : nullptr,
             static_cast<uint16_t*>(c.data_ptr()), M, N, K, scale.has_value() ? 1 : 0, bias.has_value() ? 1 : 0,
             static_cast<const uint16_t*>(lora_t.data_ptr()), static_cast<const uint16_t*>(lora_u.data_ptr()), R,
-            lora_t.scalar_type() == at::kHalf ? FEATHER_DTYPE_F16 : FEATHER_DTYPE_BF16, cfg[0], cfg[1], cfg[2],
-            cfg[3], cfg[4], b_dtype, out_dtype == at::kHalf ? 0 : 1, stream);
-        if (launched) return c;
+            lora_t.scalar_type() == at::kHalf ? FEATHER_DTYPE_F16 : FEATHER_DTYPE_BF16, b_dtype,
+            out_dtype == at::kHalf ? 0 : 1, ws, ws_size, stream);
+    };
+    at::Tensor x = a;
+    if (launch(a, a.scalar_type() == at::kHalf ? FEATHER_DTYPE_F16 : FEATHER_DTYPE_BF16)) return c;
+    if (a.scalar_type() == at::kBFloat16 && b_dtype == 1) {  // the tiles take fp16 activations
+        x = at::empty(a.sizes(), a.options().dtype(at::kHalf));
+        const int st = feather_bf16_to_fp16_rne(static_cast<const uint16_t*>(a.data_ptr()),
+                                                static_cast<uint16_t*>(x.data_ptr()), a.numel(), stream);
+        TORCH_CHECK(st == FEATHER_OK, "feather_bf16_to_fp16_rne failed: ", feather_status_string(st));
+        if (launch(x, FEATHER_DTYPE_F16)) return c;
     }
-    at::Tensor c = scaled_mm_any_m(a, b_prepacked, scale, bias, out_dtype);
+    c = scaled_mm_any_m(x, b_prepacked, scale, bias, out_dtype);
     c.add_(at::mm(lora_t, lora_u.t()).to(out_dtype));
     return c;
 }

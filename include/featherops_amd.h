@@ -126,6 +126,23 @@ bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b
                                     size_t workspace_bytes, hipStream_t stream);
 
 /*
+ * feather_launch_scaled_mm_any_m plus the unmerged-LoRA term T . U^T (arguments as
+ * feather_launch_scaled_mm_lora's). On shapes that the tuple route serves with a large
+ * tile the term joins the scaled fp32 accumulator; elsewhere it is rounded to the
+ * factors' type and to the output type and added to the finished result in the output
+ * type, as a separate pass would. Returns false and launches nothing where no kernel
+ * adds the term (e4m3fn weights; bf16 activations beyond the small-M kernel; K % 64
+ * != 0 on the widest grids). Workspace: the size below, the contract of
+ * feather_launch_scaled_mm_ws.
+ */
+size_t feather_scaled_mm_any_m_lora_workspace_size(int64_t M, int64_t N, int64_t K);
+bool feather_launch_scaled_mm_any_m_lora(const void* a, int a_dtype, const uint8_t* b_prepacked, const float* scale,
+                                         const uint16_t* bias, uint16_t* c, int64_t M, int64_t N, int64_t K,
+                                         int has_scale, int has_bias, const uint16_t* lora_t, const uint16_t* lora_u,
+                                         int64_t rank, int lora_dtype, int b_dtype, int output_dtype, void* workspace,
+                                         size_t workspace_bytes, hipStream_t stream);
+
+/*
  * feather_launch_scaled_mm_ex without a workspace argument and without any
  * allocation. No counterpart in the reference: it is for callers that cannot
  * allocate device memory -- code under HIP graph capture, tight serving

@@ -59,3 +59,48 @@ def test_planned_tile(cuda, hk, M, N, K, kid, split, b_dtype, out_dtype):
     ref = torch_ref_dev(a, bp, s, None, out_dtype, b_dtype=b_dtype)
     y = hk.scaled_mm_hip_any_m(a, bp, s, None, out_dtype)
     assert_gemm_close_dev(y, ref, out_dtype, f"{M}x{N}x{K} kernel {kid} non-finite")
+
+
+# (M, N, K): one per planned tile and per place of the term's rounding, K splits, the lean small-M kernel (one and two
+# row tiles), and the routes without a fused term
+LORA_SHAPES = [
+    (1, 4096, 1024), (16, 528, 512), (5, 13824, 5120), (31, 2048, 2048), (17, 1040, 1024),
+    (63, 224, 128), (33, 128, 2480), (130, 5488, 128), (17, 5456, 5648), (333, 1712, 3904), (33, 2864, 4464),
+    (333, 2976, 1664), (65, 3776, 5040), (777, 2160, 2816), (97, 4160, 3984), (333, 5408, 1728), (200, 4640, 5520),
+    (500, 4416, 2368), (200, 5504, 4528), (1003, 4304, 896), (777, 5056, 4880), (1003, 1632, 128), (777, 4064, 2704),
+    (777, 4928, 64), (1300, 3536, 2096), (2000, 3712, 4528), (2000, 6160, 128), (1300, 4640, 128), (2000, 4352, 1408),
+    (2000, 4832, 128), (8, 2048, 12288),
+]
+
+
+@pytest.mark.parametrize("out_dtype,f_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
+                                               (torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)])
+@pytest.mark.parametrize("M,N,K", LORA_SHAPES)
+def test_planned_tile_lora(cuda, hk, M, N, K, out_dtype, f_dtype):
+    """The rank-R term on every planned tile, against the whole output in float64 with the term in the
+    accumulator (tuple route on a large tile) or rounded and added to the result (every other)."""
+    R = 32 * (1 + (M + N // 16) % 5)
+    g = torch.Generator(device=cuda).manual_seed(M + N + K + 1)
+    a = torch.randn(M, K, generator=g, device=cuda).half()
+    w = torch.randn(N, K, generator=g, device=cuda) * 0.02
+    s = (w.abs().max() / 57344.0).float().reshape(1)
+    bp = (w / s).to(torch.float8_e5m2).view(N, K // 16, 16).permute(1, 0, 2).contiguous()
+    bias = (torch.randn(N, generator=g, device=cuda) * 0.1).to(out_dtype)
+    t = (torch.randn(M, R, generator=g, device=cuda) * 0.2).to(f_dtype)
+    u = (torch.randn(N, R, generator=g, device=cuda) * 0.05).to(f_dtype)
+    print("planned tile, rank", R, "term", M, N, K, out_dtype, f_dtype, flush=True)
+    y = hk.scaled_mm_hip_any_m_lora(a, bp, s, bias, out_dtype, t, u)
+    term = t.double() @ u.double().t()
+    if 20 <= hk.kernel_id(M, N, K, hk.any_m_config(M, N, K)) < 30:
+        dec = bp.double().permute(0, 2, 1).reshape(K, N)
+        ref = (((a.double() @ dec) * s.double() + term).to(out_dtype).float() + bias.float()).to(out_dtype)
+    else:
+        ref = torch_ref_dev(a, bp, s, bias, out_dtype)
+        ref = (ref.float() + term.to(f_dtype).to(out_dtype).float()).to(out_dtype)
+    assert_gemm_close_dev(y, ref, out_dtype, f"{M}x{N}x{K} rank {R}")
+    y2 = hk.scaled_mm_hip_any_m_lora(a, bp, s, bias, out_dtype, t, u)
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+    ab = a.bfloat16()  # bf16 activations: the bits of their fp16 cast
+    yb = hk.scaled_mm_hip_any_m_lora(ab, bp, s, bias, out_dtype, t, u)
+    y16 = hk.scaled_mm_hip_any_m_lora(ab.half(), bp, s, bias, out_dtype, t, u)
+    assert torch.equal(yb.view(torch.int16), y16.view(torch.int16))
