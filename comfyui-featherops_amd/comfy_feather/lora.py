@@ -79,6 +79,32 @@ def lora_factors(x: torch.Tensor, weight_functions, cache: dict | None = None):
     the same tensor objects, unmodified in place (version counters), with the
     same strengths, and x has the same dtype and device; the entry keeps the
     tensors themselves, so their ids cannot be recycled while it lives."""
+    factors = _factor_matrices(x, weight_functions, cache)
+    if factors is None:
+        return None
+    d, u = factors
+    return lora_down(x, d), u
+
+
+def lora_layer_inputs(x: torch.Tensor, weight_functions, cache: dict | None = None):
+    """lora_factors(x, ...) and the activations the GEMM should be given: (T, U, x'), or None.
+    For bf16 x of more than 48 rows the GEMM takes fp16 activations, so with at most 128
+    ranks x' is x.to(float16) from the down-projection's own pass over x (the small-M kernel
+    that serves fewer rows takes bf16); otherwise x' is x."""
+    factors = _factor_matrices(x, weight_functions, cache)
+    if factors is None:
+        return None
+    d, u = factors
+    if (x.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] > 48 and d.shape[0] <= 128 and x.is_cuda
+            and x.shape[1] % 16 == 0 and x.shape[1] < (1 << 22) and x.is_contiguous()
+            and x.data_ptr() % 16 == 0 and d.data_ptr() % 16 == 0):
+        _lib.load_torch_ops()
+        t, x16 = torch.ops.feather_ops.lora_down_cast.default(x, d)
+        return t, u, x16
+    return lora_down(x, d), u, x
+
+
+def _factor_matrices(x: torch.Tensor, weight_functions, cache: dict | None):
     if x.dtype not in (torch.float16, torch.bfloat16):
         return None
     patches = _basic_patches(weight_functions)
@@ -95,7 +121,7 @@ def lora_factors(x: torch.Tensor, weight_functions, cache: dict | None = None):
         else:
             d, u = _stacked_factors(x, patches)
             cache["entry"] = (key, [(dn, up) for dn, up, _ in patches], d, u)
-    return lora_down(x, d), u
+    return d, u
 
 
 def lora_down(x: torch.Tensor, d: torch.Tensor) -> torch.Tensor:

@@ -25,7 +25,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from ..kernel.hip.hip_kernel import scaled_mm_hip, scaled_mm_hip_any_m, scaled_mm_hip_any_m_lora
-from .lora import apply_lora_patches, lora_factors
+from .lora import apply_lora_patches, lora_layer_inputs
 from .quant import (
     HAVE_COMFY,
     get_feather_plain_tensors,
@@ -153,8 +153,8 @@ def feather_ops(out_dtype=torch.bfloat16, excluded_names=()):
             # an empty weight_function stays as it is, a used one is set aside without Module's
             # attribute write (2.2 us, twice; it holds a plain list), and reshape, to and view run
             # only where they apply.
-            def _forward_padded(self, x, lora=None):
-                dtype_orig = x.dtype
+            def _forward_padded(self, x, lora=None, dtype_orig=None):
+                dtype_orig = dtype_orig or x.dtype
                 x = x.contiguous()
                 if x.dtype != torch.float16 and (self.pad_m or x.dtype != torch.bfloat16):
                     # (bf16 activations go to the any-M entry as they are: the
@@ -210,11 +210,13 @@ def feather_ops(out_dtype=torch.bfloat16, excluded_names=()):
                     # basic LoRA patches go into the GEMM's epilogue (one pass over C)
                     if self.fuse_lora:
                         cache = self.__dict__.setdefault("_lora_factor_cache", {})
-                        lora = lora_factors(x, self.weight_function, cache)
+                        lora = lora_layer_inputs(x, self.weight_function, cache)
                     else:
                         lora = None
-                    y = self._forward_padded(x, lora)
-                    if lora is None:
+                    if lora is not None:
+                        y = self._forward_padded(lora[2], lora[:2], x.dtype)
+                    else:
+                        y = self._forward_padded(x)
                         y = apply_lora_patches(x, y, self.weight_function)
                 return y if len(shape) == 2 else y.view(*shape[:-1], y.shape[-1])
 

@@ -599,6 +599,29 @@ int feather_lora_down(const void* x, int x_dtype, const void* d, void* t, int64_
     return launch_status();
 }
 
+int feather_lora_down_cast(const void* x, const void* d, void* t, uint16_t* x16, int64_t M, int64_t K, int64_t R,
+                           void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    if (M < 0 || K <= 0 || R <= 0 || M > INT32_MAX) return FEATHER_ERR_INVALID;
+    // one rank chunk (its workgroups store each row of x once); 32-bit offsets within 128 rows
+    if (K % 8 != 0 || R % 32 != 0 || R > 128 || K >= (int64_t{1} << 23)) return FEATHER_ERR_UNSUPPORTED;
+    if (M == 0) return FEATHER_OK;
+    if (!x || !d || !t || !x16) return FEATHER_ERR_INVALID;
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(t) |
+         reinterpret_cast<uintptr_t>(x16)) % 16 != 0)
+        return FEATHER_ERR_INVALID;
+    feather::LoraDownArgs a;
+    a.x = static_cast<const uint16_t*>(x);
+    a.d = static_cast<const uint16_t*>(d);
+    a.t = static_cast<uint16_t*>(t);
+    a.x16 = x16;
+    a.M = M;
+    a.K = K;
+    a.R = R;
+    a.bf16 = true;
+    feather::launch_lora_down(a, workspace, workspace_bytes, stream);
+    return launch_status();
+}
+
 const char* feather_status_string(int status) {
     switch (status) {
         case FEATHER_OK: return "ok";

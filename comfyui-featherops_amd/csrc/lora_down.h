@@ -13,6 +13,7 @@ struct LoraDownArgs {
     uint16_t* t;        // (M, R) same dtype
     int64_t M, K, R;    // R % 32 == 0
     bool bf16;
+    uint16_t* x16 = nullptr;  // bf16 x, R <= 128: x rounded to fp16 as well, (M, K), 16-byte aligned
 };
 
 // Workspace the K split across workgroups can use (0: the call runs unsplit).

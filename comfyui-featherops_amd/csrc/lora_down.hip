@@ -26,7 +26,15 @@
 //     of the split-K GEMM tiles (device-coherent (sc1) 16-byte partial stores
 //     and loads, a vmcnt wait before the barrier that precedes the counter RMW);
 //   * rows past M read the last row (results dropped); 8-element K chunks past
-//     K are zeroed in registers on both operands.
+//     K are zeroed in registers on both operands;
+//   * kCast (bf16 x, one rank chunk): the GEMM behind it takes x in fp16, so each
+//     wave also rounds the fragments it reads (the two wave columns one K half
+//     each) and stores them: x is read once and a launch saved (whole bf16 layers:
+//     M=333 N=K=3072 rank 32 26.4 -> 22.3 us, M=4608 rank 64 86.9 -> 80.9);
+//   * operands past K are masked in a branch only the last stage takes, and a K
+//     half's fragments are all read before its first MFMA (masked at every read,
+//     each read waited for the one before: M=4608 K=3072 R=64 12.5 -> 10.5 us,
+//     M=4096 K=12288 R=64 27.2 -> 24.9, M=333 K=3072 R=32 7.2 -> 6.4).
 #include "feather_common.h"
 #include "featherops_amd.h"
 #include "lds_dma.h"
@@ -40,12 +48,13 @@ constexpr int kLdBK = 64;  // K per stage
 
 // WM x WN waves; wave (wm, wn) owns rows 32 wm .. 32 wm + 31 (two 16-row tiles) and
 // rank tiles wn * RN / WN .. of the workgroup's 32 * WM rows x 16 * RN ranks.
-template <int WM, int WN, int RN, bool kBf16, int kStagesReq>
+template <int WM, int WN, int RN, bool kBf16, int kStagesReq, bool kCast>
 __global__ __launch_bounds__(64 * WM * WN) void lora_down_kernel(const uint16_t* __restrict__ x,
                                                                   const uint16_t* __restrict__ d,
                                                                   uint16_t* __restrict__ t, int M, int K, int R,
                                                                   int r_base, int ksplit, float* __restrict__ partials,
-                                                                  uint32_t* __restrict__ counters) {
+                                                                  uint32_t* __restrict__ counters,
+                                                                  uint16_t* __restrict__ x16) {
     constexpr int kWaves = WM * WN;
     constexpr int kRows = 32 * WM;
     constexpr int RNW = RN / WN;  // rank tiles per wave
@@ -125,32 +134,61 @@ __global__ __launch_bounds__(64 * WM * WN) void lora_down_kernel(const uint16_t*
         const v4 v = *reinterpret_cast<const __attribute__((address_space(3))) v4*>(static_cast<uintptr_t>(addr));
         return make_uint4(v.x, v.y, v.z, v.w);
     };
+    // fp16 copy of this block's rows: buffer stores, which drop a lane past the last
+    // row or past K, so every wave issues the same two a stage (the wait counts below)
+    static_assert(!kCast || (kBf16 && WN == 2), "the two wave columns round one K half each");
+    [[maybe_unused]] const int64_t row_bytes = static_cast<int64_t>(K) * 2;
+    [[maybe_unused]] const int rows = M - m0 < kRows ? M - m0 : kRows;
+    const __amdgpu_buffer_rsrc_t x16_rs = __builtin_amdgcn_make_buffer_rsrc(
+        kCast ? x16 + static_cast<int64_t>(m0) * K : nullptr, 0,
+        kCast ? static_cast<int>(static_cast<uint32_t>(rows * row_bytes)) : 0, 0x00020000);
     auto compute = [&](int b, int st) {
         const uint32_t lb = lds_addr_of(sbuf[b]);
         const int kbase = (st0 + st) * kLdBK;
+        const bool past = kbase + kLdBK > K;  // uniform: only a stage that reaches past K masks its operands
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             // lane group lg holds logical chunk 2 * lg + h of every row
             const int ch = 2 * lg + h;
             const bool live = kbase + ch * 8 < K;
-            uint4 xa[2];
+            uint4 xa[2], db[RNW];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int xr = wm * 32 + i * 16 + lr;
                 xa[i] = lds_ld16(lb + xr * 128 + ((ch ^ swz(xr)) << 4));
-                if (!live) xa[i] = make_uint4(0u, 0u, 0u, 0u);
             }
 #pragma unroll
             for (int rn = 0; rn < RNW; ++rn) {
                 const int dr = (wn * RNW + rn) * 16 + lr;
-                uint4 db = lds_ld16(lb + kXStage + dr * 128 + ((ch ^ swz(dr)) << 4));
-                if (!live) db = make_uint4(0u, 0u, 0u, 0u);
+                db[rn] = lds_ld16(lb + kXStage + dr * 128 + ((ch ^ swz(dr)) << 4));
+            }
+            if (past && !live) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    if constexpr (kBf16) acc[i][rn] = mfma16x16x32_bf16(db, xa[i], acc[i][rn]);
-                    else acc[i][rn] = mfma16x16x32(as_half8(db), as_half8(xa[i]), acc[i][rn]);
+                for (int i = 0; i < 2; ++i) xa[i] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+                for (int rn = 0; rn < RNW; ++rn) db[rn] = make_uint4(0u, 0u, 0u, 0u);
+            }
+            if constexpr (kCast) {
+                if (wn == h) {
+                    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const int xr = wm * 32 + i * 16 + lr;
+                        const uint32_t off = live && xr < rows ? static_cast<uint32_t>(xr) * static_cast<uint32_t>(row_bytes) +
+                                                                     static_cast<uint32_t>(kbase + ch * 8) * 2u
+                                                               : 0xffffffffu;
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, a_frag<true>(xa[i])), x16_rs,
+                                                               static_cast<int>(off), 0, 0);
+                    }
                 }
             }
+#pragma unroll
+            for (int rn = 0; rn < RNW; ++rn)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if constexpr (kBf16) acc[i][rn] = mfma16x16x32_bf16(db[rn], xa[i], acc[i][rn]);
+                    else acc[i][rn] = mfma16x16x32(as_half8(db[rn]), as_half8(xa[i]), acc[i][rn]);
+                }
         }
     };
 
@@ -164,7 +202,16 @@ __global__ __launch_bounds__(64 * WM * WN) void lora_down_kernel(const uint16_t*
         for (int i = 0; i < kS - 1; ++i) issue_stage(i, i < nst ? i : nst - 1);
     }
     for (int st = 0; st < nst; ++st) {
-        wait_vmcnt<(kS - 2) * kLoads>();
+        // the copies of stage st are in once only what was issued after them is outstanding: the
+        // copies of kS - 2 stages and, with kCast, two stores a stage from the kS-th wait on
+        // (loads and stores retire in issue order; before that the copies' count alone is the
+        // stricter one)
+        if constexpr (kCast) {
+            if (st >= kS - 1) wait_vmcnt<(kS - 2) * (kLoads + 2) + 2>();
+            else wait_vmcnt<(kS - 2) * kLoads>();
+        } else {
+            wait_vmcnt<(kS - 2) * kLoads>();
+        }
         stage_barrier();  // stage st landed for every wave; stage st - 1's buffer is free
         const int nx = st + kS - 1;
         issue_stage(nx % kS, nx < nst ? nx : nst - 1);
@@ -198,7 +245,7 @@ __global__ __launch_bounds__(64 * WM * WN) void lora_down_kernel(const uint16_t*
         __syncthreads();
         if (!last_flag) return;
         // the splits are added in split order, kQ splits' loads in flight at a time
-        constexpr int kQ = RNW <= 1 ? 4 : RNW <= 2 ? 2 : 1;
+        constexpr int kQ = RNW <= 1 ? 8 : RNW <= 2 ? 4 : 2;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -303,14 +350,14 @@ void launch_wm(const LoraDownArgs& a, const LoraChunk& c, int ks, float* partial
     // stages measured slower on these shapes; at one to four row blocks every form is within
     // 2% and the earlier loop slightly ahead (M=16 K=3072 R=64: 54.4 vs 55.4 GB/s)
     constexpr int kS = RN <= 4 ? 4 : 3;
-    if (a.bf16)
-        hipLaunchKernelGGL((lora_down_kernel<WM, 2, RN, true, kS>), grid, block, 0, stream, a.x, a.d, a.t,
-                           static_cast<int>(a.M), static_cast<int>(a.K), static_cast<int>(a.R), c.r_base, ks, partials,
-                           counters);
-    else
-        hipLaunchKernelGGL((lora_down_kernel<WM, 2, RN, false, kS>), grid, block, 0, stream, a.x, a.d, a.t,
-                           static_cast<int>(a.M), static_cast<int>(a.K), static_cast<int>(a.R), c.r_base, ks, partials,
-                           counters);
+#define FEATHER_LORA_DOWN(BF, CAST)                                                                              \
+    hipLaunchKernelGGL((lora_down_kernel<WM, 2, RN, BF, kS, CAST>), grid, block, 0, stream, a.x, a.d, a.t,      \
+                       static_cast<int>(a.M), static_cast<int>(a.K), static_cast<int>(a.R), c.r_base, ks,      \
+                       partials, counters, a.x16)
+    if (a.bf16 && a.x16) FEATHER_LORA_DOWN(true, true);
+    else if (a.bf16) FEATHER_LORA_DOWN(true, false);
+    else FEATHER_LORA_DOWN(false, false);
+#undef FEATHER_LORA_DOWN
 }
 
 template <int RN>

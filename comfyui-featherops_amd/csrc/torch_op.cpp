@@ -10,8 +10,8 @@
 //                                 fused into the epilogue on the large tiles
 //   feather_ops::quantize_prepack_e5m2(_scaled)
 //                                 the fused quantize + prepack of a weight
-//   feather_ops::lora_down        T = F.linear(x, d), the LoRA down-projection
-//                                 of all patches at once
+//   feather_ops::lora_down(_cast) T = F.linear(x, d), the LoRA down-projection
+//                                 of all patches at once (and x in fp16)
 //   feather_ops_internal::scaled_mm_configured
 //                                 the reference's configured op (hip_kernel.py:
 //                                 12-58, a Python custom op there), Meta kernel
@@ -342,6 +342,33 @@ at::Tensor lora_down(const at::Tensor& x, const at::Tensor& d) {
     return t;
 }
 
+// feather_ops::lora_down_cast: lora_down of bf16 x (at most 128 ranks) and x.to(float16), in
+// one pass over x.
+std::tuple<at::Tensor, at::Tensor> lora_down_cast(const at::Tensor& x, const at::Tensor& d) {
+    TORCH_CHECK(x.is_cuda() && d.is_cuda() && d.device() == x.device(), "x and d must be CUDA tensors on one device");
+    TORCH_CHECK(x.dim() == 2 && d.dim() == 2 && x.size(1) == d.size(1), "x must be (M, K) and d (R, K)");
+    TORCH_CHECK(x.scalar_type() == at::kBFloat16 && d.scalar_type() == at::kBFloat16, "x and d must be bfloat16");
+    TORCH_CHECK(x.is_contiguous() && d.is_contiguous(), "x and d must be contiguous");
+    const int64_t M = x.size(0), K = x.size(1), R = d.size(0);
+    TORCH_CHECK(K % 8 == 0 && R > 0 && R % 32 == 0 && R <= 128,
+                "lora_down_cast needs K % 8 == 0 and R a multiple of 32 up to 128");
+    at::Tensor t = at::empty({M, R}, x.options());
+    at::Tensor x16 = at::empty({M, K}, x.options().dtype(at::kHalf));
+    if (M == 0) return {t, x16};
+    const c10::DeviceGuard guard(x.device());
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+    const size_t ws_bytes = feather_lora_down_workspace_size(M, K, R);
+    void* ws = ws_bytes ? workspace_for(x.device(), stream, ws_bytes).data_ptr() : nullptr;
+    const int st = feather_lora_down_cast(x.data_ptr(), d.data_ptr(), t.data_ptr(), static_cast<uint16_t*>(x16.data_ptr()),
+                                          M, K, R, ws, ws_bytes, stream);
+    TORCH_CHECK(st == FEATHER_OK, "feather_lora_down_cast failed: ", feather_status_string(st));
+    return {t, x16};
+}
+
+std::tuple<at::Tensor, at::Tensor> lora_down_cast_meta(const at::Tensor& x, const at::Tensor& d) {
+    return {at::empty({x.size(0), d.size(0)}, x.options()), at::empty(x.sizes(), x.options().dtype(at::kHalf))};
+}
+
 at::Tensor lora_down_meta(const at::Tensor& x, const at::Tensor& d) {
     return at::empty({x.size(0), d.size(0)}, x.options());
 }
@@ -452,6 +479,7 @@ TORCH_LIBRARY(feather_ops, m) {
     m.def("quantize_prepack_e5m2(Tensor w, Tensor? ckpt_scale, bool native) -> (Tensor, Tensor)");
     m.def("quantize_prepack_e5m2_scaled(Tensor w, Tensor scale) -> Tensor");
     m.def("lora_down(Tensor x, Tensor d) -> Tensor");
+    m.def("lora_down_cast(Tensor x, Tensor d) -> (Tensor, Tensor)");
     m.def("bf16_to_fp16(Tensor x, bool rne) -> Tensor");
 }
 
@@ -462,6 +490,7 @@ TORCH_LIBRARY_IMPL(feather_ops, CUDA, m) {
     m.impl("quantize_prepack_e5m2", &quantize_prepack_e5m2);
     m.impl("quantize_prepack_e5m2_scaled", &quantize_prepack_e5m2_scaled);
     m.impl("lora_down", &lora_down);
+    m.impl("lora_down_cast", &lora_down_cast);
     m.impl("bf16_to_fp16", &bf16_to_fp16);
 }
 
@@ -469,6 +498,7 @@ TORCH_LIBRARY_IMPL(feather_ops, Meta, m) {
     m.impl("scaled_mm_any_m", &scaled_mm_any_m_meta);
     m.impl("scaled_mm_any_m_lora", &scaled_mm_any_m_lora_meta);
     m.impl("lora_down", &lora_down_meta);
+    m.impl("lora_down_cast", &lora_down_cast_meta);
     m.impl("bf16_to_fp16", &bf16_to_fp16_meta);
 }
 

@@ -204,6 +204,14 @@ bool feather_launch_scaled_mm_lora(const void* a, const uint8_t* b_prepacked, co
  */
 int feather_lora_down(const void* x, int x_dtype, const void* d, void* t, int64_t M, int64_t K, int64_t R,
                       void* workspace, size_t workspace_bytes, hipStream_t stream);
+/*
+ * feather_lora_down for bf16 x that also writes x rounded to fp16 (to nearest even, the
+ * values of feather_bf16_to_fp16_rne) into x16 (M, K): one pass over x before a GEMM that
+ * takes fp16 activations. R <= 128 and K < 2^23, else FEATHER_ERR_UNSUPPORTED. Workspace as
+ * feather_lora_down's.
+ */
+int feather_lora_down_cast(const void* x, const void* d, void* t, uint16_t* x16, int64_t M, int64_t K, int64_t R,
+                           void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 /* Workspace bytes feather_lora_down can use for this call (0 = none). */
 size_t feather_lora_down_workspace_size(int64_t M, int64_t K, int64_t R);

@@ -154,3 +154,31 @@ def test_lora_down_python_entry_falls_back_on_misaligned_x(cuda, hk, pkg):
     x_al = x_off.clone()
     t_al = lora.lora_down(x_al, d)
     assert_gemm_close(t_al, O.lora_down_ref(_np(x_al), _np(d), O.DT_F16), torch.float16, "aligned x")
+
+
+@pytest.mark.parametrize("M,K,R", [(1, 8, 32), (17, 24, 64), (300, 1040, 96), (256, 3072, 128), (129, 2048, 64),
+                                   (8200, 64, 32), (4608, 3072, 64), (70, 4160, 128), (28800, 256, 32), (333, 3072, 32)])
+def test_lora_down_cast(cuda, hk, M, K, R):
+    """The down-projection that also writes x in fp16 (ragged M and K, K splits, both block heights,
+    every ring depth): T as the plain kernel's bits, the copy as x.to(float16)'s, overflow and
+    subnormals included, and nothing written past the last row."""
+    g = torch.Generator(device=cuda).manual_seed(M + K + R)
+    x = torch.randn(M, K, generator=g, device=cuda).bfloat16()
+    x[0, :3] = torch.tensor([1.0e6, 3.0e-6, -5.0e-8], device=cuda)
+    x[M - 1, K - 1] = float("-inf")
+    d = (torch.randn(R, K, generator=g, device=cuda) * 0.05).bfloat16()
+    t0 = torch.ops.feather_ops.lora_down.default(x, d)
+    nbytes = lib().feather_lora_down_workspace_size(M, K, R)
+    ws = torch.zeros(max(nbytes, 16), dtype=torch.uint8, device=cuda)
+    t = torch.full((M, R), float("nan"), dtype=torch.bfloat16, device=cuda)
+    x16 = torch.full((M + 3, K), 7.0, dtype=torch.float16, device=cuda)
+    print("lora_down_cast", M, K, R, flush=True)
+    st = lib().feather_lora_down_cast(x.data_ptr(), d.data_ptr(), t.data_ptr(), x16.data_ptr(), M, K, R,
+                                      ws.data_ptr() if nbytes else None, nbytes, stream(cuda))
+    assert st == 0, lib().feather_status_string(st)
+    torch.cuda.synchronize()
+    assert torch.equal(t.view(torch.int16), t0.view(torch.int16))
+    assert torch.equal(x16[:M].view(torch.int16), x.to(torch.float16).view(torch.int16))
+    assert (x16[M:] == 7.0).all()
+    assert lib().feather_lora_down_cast(x.data_ptr(), d.data_ptr(), t.data_ptr(), x16.data_ptr(), M, K, 160, None, 0,
+                                        stream(cuda)) != 0  # more than one rank chunk
