@@ -28,8 +28,9 @@
 //   * rows past M read the last row (results dropped); 8-element K chunks past
 //     K are zeroed in registers on both operands;
 //   * kCast (bf16 x, one rank chunk): the GEMM behind it takes x in fp16, so each
-//     wave also rounds the fragments it reads (the two wave columns one K half
-//     each) and stores them: x is read once and a launch saved (whole bf16 layers:
+//     wave also rounds the x rows it copied and stores them, in whole 128-byte runs
+//     (from the MFMA fragments, 16 bytes in 32, M=4096 K=12288 R=64 took 53 us
+//     against 45 for projection and cast): x is read once and a launch saved (whole bf16 layers:
 //     M=333 N=K=3072 rank 32 26.4 -> 22.3 us, M=4608 rank 64 86.9 -> 80.9);
 //   * operands past K are masked in a branch only the last stage takes, and a K
 //     half's fragments are all read before its first MFMA (masked at every read,
@@ -135,17 +136,29 @@ __global__ __launch_bounds__(64 * WM * WN) void lora_down_kernel(const uint16_t*
         return make_uint4(v.x, v.y, v.z, v.w);
     };
     // fp16 copy of this block's rows: buffer stores, which drop a lane past the last
-    // row or past K, so every wave issues the same two a stage (the wait counts below)
-    static_assert(!kCast || (kBf16 && WN == 2), "the two wave columns round one K half each");
-    [[maybe_unused]] const int64_t row_bytes = static_cast<int64_t>(K) * 2;
+    // row or past K, so every wave issues the same kXPerWave a stage (the wait counts below)
+    static_assert(!kCast || kBf16, "the fp16 copy is of bf16 x");
+    [[maybe_unused]] const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
     [[maybe_unused]] const int rows = M - m0 < kRows ? M - m0 : kRows;
     const __amdgpu_buffer_rsrc_t x16_rs = __builtin_amdgcn_make_buffer_rsrc(
         kCast ? x16 + static_cast<int64_t>(m0) * K : nullptr, 0,
-        kCast ? static_cast<int>(static_cast<uint32_t>(rows * row_bytes)) : 0, 0x00020000);
+        kCast ? static_cast<int>(static_cast<uint32_t>(rows) * row_bytes) : 0, 0x00020000);
     auto compute = [&](int b, int st) {
         const uint32_t lb = lds_addr_of(sbuf[b]);
         const int kbase = (st0 + st) * kLdBK;
         const bool past = kbase + kLdBK > K;  // uniform: only a stage that reaches past K masks its operands
+        if constexpr (kCast) {
+            // the rows this wave copied, in the copies' order: eight rows of 128 bytes a store
+#pragma unroll
+            for (int i = 0; i < kXPerWave; ++i) {
+                typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+                const half8_t c = a_frag<true>(lds_ld16(lb + ldst[i] + lane * 16));
+                const int row = (i * kWaves + wave) * 8 + (lane >> 3);
+                const uint32_t kb = static_cast<uint32_t>(kbase) * 2u + coff[i];
+                const uint32_t off = row < rows && kb < row_bytes ? static_cast<uint32_t>(row) * row_bytes + kb : 0xffffffffu;
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, c), x16_rs, static_cast<int>(off), 0, 0);
+            }
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             // lane group lg holds logical chunk 2 * lg + h of every row
@@ -168,20 +181,6 @@ __global__ __launch_bounds__(64 * WM * WN) void lora_down_kernel(const uint16_t*
 #pragma unroll
                 for (int rn = 0; rn < RNW; ++rn) db[rn] = make_uint4(0u, 0u, 0u, 0u);
             }
-            if constexpr (kCast) {
-                if (wn == h) {
-                    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        const int xr = wm * 32 + i * 16 + lr;
-                        const uint32_t off = live && xr < rows ? static_cast<uint32_t>(xr) * static_cast<uint32_t>(row_bytes) +
-                                                                     static_cast<uint32_t>(kbase + ch * 8) * 2u
-                                                               : 0xffffffffu;
-                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, a_frag<true>(xa[i])), x16_rs,
-                                                               static_cast<int>(off), 0, 0);
-                    }
-                }
-            }
 #pragma unroll
             for (int rn = 0; rn < RNW; ++rn)
 #pragma unroll
@@ -203,11 +202,11 @@ __global__ __launch_bounds__(64 * WM * WN) void lora_down_kernel(const uint16_t*
     }
     for (int st = 0; st < nst; ++st) {
         // the copies of stage st are in once only what was issued after them is outstanding: the
-        // copies of kS - 2 stages and, with kCast, two stores a stage from the kS-th wait on
+        // copies of kS - 2 stages and, with kCast, kXPerWave stores a stage from the kS-th wait on
         // (loads and stores retire in issue order; before that the copies' count alone is the
         // stricter one)
         if constexpr (kCast) {
-            if (st >= kS - 1) wait_vmcnt<(kS - 2) * (kLoads + 2) + 2>();
+            if (st >= kS - 1) wait_vmcnt<(kS - 2) * (kLoads + kXPerWave) + kXPerWave>();
             else wait_vmcnt<(kS - 2) * kLoads>();
         } else {
             wait_vmcnt<(kS - 2) * kLoads>();
@@ -308,17 +307,25 @@ int lora_chunks(int64_t R, LoraChunk out[2]) {
 int lora_rows(int64_t M, int nchunks) { return (M + 127) / 128 * nchunks >= 224 ? 128 : 64; }
 
 // K split for this launch: as many splits as keep the grid within one
-// workgroup per CU (at most 16, at least two stages per split). Rounding the
+// workgroup per CU (at least two stages per split). Rounding the
 // split count down rather than up: M=4608 K=3072 R=64 (72 row blocks, 216 vs
-// 288 workgroups) 2435 vs 2315 GB/s on the four-stage ring.
-int lora_ksplit(int64_t M, int64_t K, int nchunks) {
+// 288 workgroups) 2435 vs 2315 GB/s on the four-stage ring. The last arriver re-reads every
+// split's partial tile, which grows with the ranks, so a split also has to be worth it: up to 8
+// splits of 32 ranks or 6 of more, more only for long K, fewer than a split a four stages
+// (us, 16 -> this rule's splits: M=1000 K=3072 R=64 12.2 -> 8.5, R=128 18.4 -> 12.7, M=333
+// K=3072 R=32 6.4 -> 5.6, M=120 K=1024 R=128 9.3 -> 8.2, M=2048 K=3072 R=64 10.2 -> 9.3).
+int lora_ksplit(int64_t M, int64_t K, int nchunks, int rn) {
     const int rows = lora_rows(M, nchunks);
     const int64_t tiles = (M + rows - 1) / rows * nchunks;
     const int64_t nst = (K + kLdBK - 1) / kLdBK;
     if (tiles > kWorkspaceCounters) return 1;
     int64_t ks = 256 / tiles;
     if (ks > nst / 2) ks = nst / 2;
-    if (ks > 16) ks = 16;
+    int64_t most = rn <= 2 ? (nst / 4 < 8 ? nst / 4 : 8) : (nst / 4 < 6 ? nst / 4 : 6);
+    const int64_t longk = nst / (rn <= 2 ? 8 : 16);
+    if (most < longk) most = longk < 16 ? longk : 16;
+    if (most < 2) most = 2;
+    if (ks > most) ks = most;
     if (ks <= 1) return 1;
     // the kernel gives split q the stages [q * per, min((q + 1) * per, nst)):
     // drop trailing splits that would own none (K = 4160: 65 stages, 16 splits
@@ -329,7 +336,7 @@ int lora_ksplit(int64_t M, int64_t K, int nchunks) {
 }
 
 size_t chunk_workspace(int64_t M, int64_t K, const LoraChunk& c) {
-    const int ks = lora_ksplit(M, K, c.nchunks);
+    const int ks = lora_ksplit(M, K, c.nchunks, c.rn);
     if (ks <= 1) return 0;
     const int rows = lora_rows(M, c.nchunks);
     const int64_t tiles = (M + rows - 1) / rows * c.nchunks;
@@ -385,7 +392,7 @@ void launch_lora_down(const LoraDownArgs& a, void* workspace, size_t workspace_b
     const int n = lora_chunks(a.R, cs);
     for (int i = 0; i < n; ++i) {
         const LoraChunk& c = cs[i];
-        int ks = lora_ksplit(a.M, a.K, c.nchunks);
+        int ks = lora_ksplit(a.M, a.K, c.nchunks, c.rn);
         const size_t need = chunk_workspace(a.M, a.K, c);
         if (ks > 1 && (workspace == nullptr || workspace_bytes < need)) ks = 1;  // no room: unsplit
         uint32_t* counters = ks > 1 ? static_cast<uint32_t*>(workspace) : nullptr;
