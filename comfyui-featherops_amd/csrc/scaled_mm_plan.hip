@@ -65,7 +65,8 @@ double cost_us(const TileCost& t, int64_t tiles, int64_t stages, int ks, int cus
 }
 
 // Small-M kernel, 17..48 rows. Up to 32: the lean kernel on unsplit 16-column strips
-// (fit of 23 shapes, 11% rms; its split plans lose to the 32-row tiles: M=22 N=1152
+// (K % 64 == 0: fit of 29 shapes, 3.5% rms; otherwise the general kernel on those strips,
+// of 23 shapes, 11% rms; the split plans lose to the 32-row tiles: M=22 N=1152
 // K=10304 12.0 vs 8.6 us, M=19 N=8576 K=6144 15.3 vs 11.8). 33..48 rows: unsplit
 // strips with K < 2048 (M=34 N=1792 K=1392 4.8 vs 5.4 us; longer K: M=38 N=2176
 // K=6848 14.8 vs 9.1).
@@ -73,6 +74,9 @@ double smallm_us(int64_t M, int64_t N, int64_t K, int cus) {
     const double mb = static_cast<double>(N) * static_cast<double>(K) * 1e-6;
     const double rounds = static_cast<double>(ceil_div(ceil_div(N, 16), cus));
     const double steps = rounds * static_cast<double>(ceil_div(K, 64));
+    if (M <= 32 && K % 64 == 0)
+        return 1.78 + 0.706 * static_cast<double>(ceil_div(N, 16)) / cus + (0.0178 + 0.0012 * static_cast<double>(M)) * steps +
+               0.0095 * mb;
     if (M <= 32) return 2.16 + 0.13 * rounds + (0.0347 + 0.0011 * static_cast<double>(M - 17)) * steps + 0.071 * mb;
     if (M <= 48 && K < 2048)
         return 1.02 + 0.63 * rounds + (0.108 + 0.0017 * static_cast<double>(M - 33)) * steps + 0.40 * mb;
@@ -89,10 +93,9 @@ MmPlan make_plan(int64_t M, int64_t N, int64_t K, int cus, bool lora) {
     MmPlan best;
     const bool lean = M <= 32 && smallm_is_lean(M, N, K, cus, M <= 16);
     if (M <= 16 && (!lora || lean)) {
-        // one row tile: the small-M kernel and its own plan. The 32 x 64 tile took up to 13%
-        // less on 11 of 70 shapes, all with wide weights (M=16 N=13824 K=5120 13.2 vs 14.3
-        // us, M=1 N=12288 K=3072 8.7 vs 10.0), but bf16 activations would need a cast pass
-        // of 3.5 us first, and both types take one plan
+        // one row tile: the small-M kernel and its own plan. The 32 x 64 tile took up to 8%
+        // less on a few wide weights (M=16 N=13824 K=5120 13.2 vs 14.3 us), but bf16
+        // activations would need a cast pass of 3.5 us first, and both types take one plan
         best.tile = kSmallM;
         best.ksplit = smallm_ksplit(M, N, K, cus);
         best.workspace_bytes = smallm_workspace_bytes(M, N, K, cus);

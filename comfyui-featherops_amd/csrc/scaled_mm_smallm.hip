@@ -257,12 +257,23 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_smallm_kernel(
 //     measured ~0.4 us slower at M=16, K=N=4096).
 // M=16, K=N=4096, 24 rotated weights, back-to-back launches: 5.87 us against
 // 6.45 us for the general kernel on the same box.
+// kPair: two workgroups share a CU (64 KB of LDS and at most 64 VGPRs each): half
+// the stages in flight per wave, and the reduction overlays the slabs. A grid
+// larger than the CU count then has one workgroup's launch, first loads and
+// reduction under the other's stream, where one workgroup per CU (145 KB) leaves
+// the memory idle between rounds: M=1 N=12288 K=3072 9.99 -> 8.25 us, M=4 N=4736
+// K=2048 4.27 -> 3.36, M=6 N=5504 K=9600 12.7 -> 10.9, M=12 N=6464 K=4672 9.6 ->
+// 8.0. With one workgroup per CU at most, the deeper form streams as fast or
+// faster (M=16 N=K=4096 5.16 vs 6.03 us, M=13 N=3520 K=4096 4.86 vs 5.84; short K
+// the other way by under 4%), so one row tile takes it there. Two row tiles are
+// always this form (M=20 N=K=4096 6.0 -> 5.6 us, M=18 N=3712 K=11392 10.7 -> 9.5,
+// M=24 N=8192 K=2048 7.1 -> 6.3; at most 3% slower, M=30 N=1792 K=2112 3.76 vs 3.87).
 // kLora: adds the rank-R term T . U^T (T (M, R), U (N, R), fp16 or bf16 by lora_bf16,
 // R % 32 == 0) to the finished result in the output type: wave t multiplies row tile
 // t's 16 x 16 product (fp32 MFMA sums, rounded to the factors' type and to the output
 // type) after its share of the stream, while the other waves write their sums.
-template <int MT, bool kBf16, bool kE4m3, bool kABf16, bool kLora>
-__global__ __launch_bounds__(64 * kWaves) void scaled_mm_m16_kernel(const uint16_t* __restrict__ A,
+template <int MT, bool kPair, bool kBf16, bool kE4m3, bool kABf16, bool kLora>
+__global__ __launch_bounds__(64 * kWaves, kPair ? 8 : 4) void scaled_mm_m16_kernel(const uint16_t* __restrict__ A,
                                                                      const uint8_t* __restrict__ Bp,
                                                                      const float* __restrict__ scale,
                                                                      const uint16_t* __restrict__ bias,
@@ -271,15 +282,16 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_m16_kernel(const uint16
                                                                      const uint16_t* __restrict__ lora_t,
                                                                      const uint16_t* __restrict__ lora_u,
                                                                      int lora_rank, int lora_bf16) {
-    constexpr int U = 4 / MT;  // stages in flight per wave (the slabs fill 128 KB of LDS)
+    constexpr int U = (kPair ? 2 : 4) / MT;  // stages in flight per wave (64 or 128 KB of slabs)
     constexpr int kStageSlab = MT * kSlabTile;
     constexpr int kRedStride = 17;
     static_assert(kWaves * 16 * MT * kRedStride * 4 <= kWaves * U * kStageSlab, "reduction fits the slabs");
     __shared__ __attribute__((aligned(1024))) uint8_t smem[kWaves * U * kStageSlab];
-    // one row tile: the cross-wave reduction buffer beside the slabs (17 KB;
-    // 145 KB in all), so a wave writes its sums as soon as it is done; two
-    // row tiles overlay it on the slabs (there is no room beside them)
-    constexpr bool kOwnRed = MT == 1;
+    // one workgroup per CU: the cross-wave reduction buffer beside the slabs (17 KB;
+    // 145 KB in all), so a wave writes its sums as soon as it is done; with two it
+    // overlays the slabs (there is no room beside them)
+    constexpr bool kOwnRed = !kPair;
+    static_assert(kPair || MT == 1, "two row tiles run as a pair");
     __shared__ __attribute__((aligned(16))) float red_own[kOwnRed ? kWaves * 16 * MT * kRedStride : 1];
     __shared__ __attribute__((aligned(16))) uint16_t term[kLora ? MT * 16 * 16 : 1];  // the rank-R term in the output type, [row][column]
     const int tid = threadIdx.x;
@@ -357,8 +369,7 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_m16_kernel(const uint16
             // (the compiler waits for the weight registers itself; the explicit
             // wait covers the copies, which it does not see). M=16 K=N=4096, 24
             // rotated weights, back to back: 5.88 vs 6.07 us (M=1 5.36 vs 5.48
-            // us); two row tiles (U = 2) measured slower this way (8.58 vs 8.34
-            // us at M=32) and wait for the whole round
+            // us)
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 braw[u] = *reinterpret_cast<const uint4*>(bcol + static_cast<int64_t>(base + u * kWaves) * 4 * kg_stride);
@@ -426,12 +437,12 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_m16_kernel(const uint16
     }
 }
 
-template <int MT>
+template <int MT, bool kPair>
 bool launch_m16(const MmArgs& p, hipStream_t stream) {
     const dim3 grid(static_cast<uint32_t>(p.N / 16));
     const dim3 block(64 * kWaves);
 #define FEATHER_M16_LAUNCH_L(BF, E4, AB, LORA)                                                                   \
-    hipLaunchKernelGGL((scaled_mm_m16_kernel<MT, BF, E4, AB, LORA>), grid, block, 0, stream, p.a, p.b, p.scale,     \
+    hipLaunchKernelGGL((scaled_mm_m16_kernel<MT, kPair, BF, E4, AB, LORA>), grid, block, 0, stream, p.a, p.b, p.scale, \
                        p.bias, p.c, static_cast<int>(p.M), static_cast<int>(p.N), static_cast<int>(p.K),            \
                        p.has_scale, p.has_bias, p.lora_t, p.lora_u, static_cast<int>(p.lora_rank),                  \
                        p.lora_dtype == 2 ? 1 : 0)
@@ -512,10 +523,10 @@ struct SmallmPlan {
 };
 
 // Cost model for M <= 32, in microseconds, from MI355X runs with rotated
-// weights. A workgroup holds 128 KB of LDS, so one runs per CU and a grid
-// larger than the CU count runs in rounds; each wave keeps a fixed number of
-// 16-byte weight loads in flight, so a workgroup streams at a rate bounded by
-// its bytes in flight over the loaded HBM latency. For one row tile (M <= 16)
+// weights. A workgroup holds 128 KB of LDS (but see kPair), so one runs per CU
+// and a grid larger than the CU count runs in rounds; each wave keeps a fixed
+// number of 16-byte weight loads in flight, so a workgroup streams at a rate
+// bounded by its bytes in flight over the loaded HBM latency. For one row tile (M <= 16)
 // the terms are fitted per kernel: a fixed cost, a cost per round (launch,
 // first-load latency, reduction, epilogue; a K split adds its partials and
 // arrival counter here), a cost per KB one CU streams that grows with the rows
@@ -524,7 +535,8 @@ struct SmallmPlan {
 // weight per ~0.052 us, a 64-column strip (twice the loads in flight) per
 // ~0.027 us, ~3.1 us per round, a whole-chip ceiling of ~7 TB/s, and ~2.6 us
 // for a K split across workgroups.
-double smallm_cost_us(int64_t M, int64_t N, int64_t nst, int ct, int ks, int cus) {
+double smallm_cost_us(int64_t M, int64_t N, int64_t K, int ct, int ks, int cus) {
+    const int64_t nst = (K + 63) / 64;
     const int64_t nstrips = (N + 16 * ct - 1) / (16 * ct);
     const int64_t groups = nstrips * ks;
     const int64_t rounds = (groups + cus - 1) / cus;
@@ -534,14 +546,21 @@ double smallm_cost_us(int64_t M, int64_t N, int64_t nst, int ct, int ks, int cus
     if (M <= 16) {
         // one row tile: least-squares fits of measured back-to-back times
         // (M = 1..16, N = 2048..13824, K = 5120..16384), one per kernel: the
-        // lean kernel (16-column strips, no split), the general kernel with
-        // 16-column strips split over K, and 64-column strips split over K
+        // lean kernel (16-column strips, no split) with one workgroup per CU
+        // and with two (46 shapes of more strips than CUs; its rounds hold twice
+        // as many), the general kernel with 16-column strips split over K, and
+        // 64-column strips, unsplit and split over K. Of the 46 shapes the choice
+        // costs 0.5% over the best of each, 5% at most (M=16 N=12288 K=3072 9.9 on
+        // wide strips, 9.4 as a pair; M=16 N=13824 K=5120 14.3 and 16.2)
         struct Fit { double c0, round, kb, kb_row, mb; };
         constexpr Fit kLean{0.05, 1.80, 0.0213, 0.0012, 0.086};
+        constexpr Fit kLeanPair{1.12, 0.83, 0.0080, 0.0013, 0.0881};
         constexpr Fit kStripSplit{1.51, 2.70, 0.0184, 0.0009, 0.122};
+        constexpr Fit kWide{0.0, 3.0, 0.0064, 0.0003, 0.100};
         constexpr Fit kWideSplit{2.57, 2.99, 0.0108, 0.0003, 0.116};
-        const Fit& f = ct >= 4 ? kWideSplit : ks > 1 ? kStripSplit : kLean;
-        return f.c0 + f.round * static_cast<double>(rounds) + (f.kb + f.kb_row * static_cast<double>(M)) * work +
+        const bool pair = ct == 1 && ks == 1 && groups > cus && K % 64 == 0;
+        const Fit& f = ct >= 4 ? (ks > 1 ? kWideSplit : kWide) : ks > 1 ? kStripSplit : pair ? kLeanPair : kLean;
+        return f.c0 + f.round * static_cast<double>(pair ? (rounds + 1) / 2 : rounds) + (f.kb + f.kb_row * static_cast<double>(M)) * work +
                f.mb * mb;
     }
     const double per_kb = ct >= 4 ? 0.027 : 0.052;
@@ -568,10 +587,10 @@ SmallmPlan smallm_plan(int64_t M, int64_t N, int64_t K, int target_groups, bool 
         if (ks > max_ks) ks = max_ks;
         pl = ks > 1 ? SmallmPlan{pl.ct, static_cast<int>(ks)} : SmallmPlan{1, 1};
     } else {
-        double best = smallm_cost_us(M, N, nst, 1, 1, cus);
+        double best = smallm_cost_us(M, N, K, 1, 1, cus);
         for (int ct : {1, 4})
             for (int ks = 1; ks <= max_ks; ++ks) {
-                const double c = smallm_cost_us(M, N, nst, ct, ks, cus);
+                const double c = smallm_cost_us(M, N, K, ct, ks, cus);
                 if (c < best) {
                     best = c;
                     pl = SmallmPlan{ct, ks};
@@ -630,8 +649,10 @@ bool launch_smallm_kernel(const MmArgs& p, void* workspace, size_t workspace_byt
     const bool wide = pl.ct >= 2;
     // A through LDS needs every byte offset into A to fit the copy's 32-bit lane offset
     const bool lds_a = p.M * p.K * 2 < (int64_t(1) << 32);
-    if (mt <= 2 && ks == 1 && !wide && lds_a && p.K % 64 == 0 && p.N % 16 == 0 && !m16_disabled())
-        return mt == 1 ? launch_m16<1>(p, stream) : launch_m16<2>(p, stream);
+    if (mt <= 2 && ks == 1 && !wide && lds_a && p.K % 64 == 0 && p.N % 16 == 0 && !m16_disabled()) {
+        if (mt == 2) return launch_m16<2, true>(p, stream);
+        return p.N / 16 > target ? launch_m16<1, true>(p, stream) : launch_m16<1, false>(p, stream);
+    }
     if (p.lora_dtype != 0) return false;  // only the lean kernel adds a rank-R term
     switch (mt) {
         case 1:
