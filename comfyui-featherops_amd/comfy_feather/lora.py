@@ -12,7 +12,7 @@ Two forms:
     by the library's down-projection kernel (lora_down), and
     U = [up_i]_i (N, R), stacked over the patches along the rank and
     zero-padded to a multiple of 32, in x's dtype. The GEMM then adds T . U^T
-    to its fp32 accumulator before rounding, so C is written once.
+    in its epilogue, so C is written once.
 """
 
 import torch

@@ -118,10 +118,13 @@ int splitk_env() {
 //     workgroups (each holds a CU's LDS, so a larger grid runs twice):
 //     M=154 N=10240 K=4096 19.9 us vs 32.0 us on 128 x 128 tiles, M=512
 //     N=3072 K=12288 47 vs 85 us, M=1024 N=2048 K=8192 36 vs 54 us, M=2048
-//     N=K=1024 7.4 vs 10.8 us; past it the tile kernel wins (M=256 N=10240
+//     N=K=1024 7.4 vs 10.8 us; past it the tuple's tile wins (M=256 N=10240
 //     K=4096: 320 workgroups, 38.2 vs 32.7 us; M=768 N=K=3072 27.4 vs 22.5 us,
 //     M=512 N=K=5120 44.8 vs 39.0 us, M=256 N=13824 K=5120 49.3 vs 41.2 us).
-// Measured on MI355X with the C++ bench. FEATHEROPS_SPLITK (tuning knob, read
+// Measured on MI355X with the C++ bench, the split-K tiles on one group of waves
+// per workgroup (two groups, as now, take 4-18% less on them). The tuple entries keep
+// this rule and its workspace sizes; the any-M entries take the cost table's plan
+// instead, unless the knob below is set. FEATHEROPS_SPLITK (tuning knob, read
 // on every call so that tests can reach the tuple's tile kernels at small
 // shapes): 0 = never, 1 = always (K % 64 == 0).
 int splitk_route(int64_t M, int64_t N, int64_t K) {

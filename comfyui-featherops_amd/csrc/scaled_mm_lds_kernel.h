@@ -3,7 +3,7 @@
 //
 // Same contract as the reference kernel (kernel/hip/hip_kernel.cu:133-420:
 // fp32 accumulation, scale on the accumulator, rounding to the output type,
-// bias added in the output type) for K % 64 == 0.
+// bias added in the output type) for K % 64 == 0, and with kTail for any K % 16.
 //
 // How it works:
 //   * global -> LDS copies use gfx950's global_load_lds_dwordx4: each wave

@@ -2,12 +2,12 @@
 // torch's dispatcher straight to the launch entry without a Python frame:
 //   feather_ops::scaled_mm        the reference's op (kernel/hip/hip_kernel.cu:
 //                                 746-767: same namespace, schema, CUDA key)
-//   feather_ops::scaled_mm_any_m  any M, shape-picked tile, fp16/bf16 A (no
+//   feather_ops::scaled_mm_any_m  any M, planned tile, fp16/bf16 A (no
 //                                 counterpart in the reference; Meta kernel for
 //                                 fake tensors)
 //   feather_ops::scaled_mm_any_m_lora
 //                                 the any-M op plus an unmerged-LoRA term,
-//                                 fused into the epilogue on the large tiles
+//                                 fused into the epilogue
 //   feather_ops::quantize_prepack_e5m2(_scaled)
 //                                 the fused quantize + prepack of a weight
 //   feather_ops::lora_down(_cast) T = F.linear(x, d), the LoRA down-projection
@@ -171,10 +171,11 @@ void scaled_mm(const at::Tensor& a, const at::Tensor& b_prepacked, const std::op
 }
 
 // feather_ops::scaled_mm_any_m: any row count M without padding (the kernels
-// mask rows past M), the tile from feather_scaled_mm_pick_config, fp16 or bf16
+// mask rows past M), tile and K split from the any-M plan, fp16 or bf16
 // activations. bf16 activations are rounded to fp16 inside the small-M kernel,
 // otherwise by the library's round-to-nearest-even cast first: the values of
-// x.to(float16) (comfy_feather/ops.py:88) either way.
+// x.to(float16) (comfy_feather/ops.py:88) either way. The argument checks and
+// their messages are those of the tuple feather_scaled_mm_pick_config names.
 at::Tensor scaled_mm_any_m(const at::Tensor& a, const at::Tensor& b_prepacked, const std::optional<at::Tensor>& scale,
                            const std::optional<at::Tensor>& bias, at::ScalarType out_dtype) {
     TORCH_CHECK(a.dim() == 2, "a must be 2D");

@@ -308,7 +308,7 @@ def any_m_config(M: int, N: int, K: int, device: torch.device | None = None) -> 
 
 # torch.ops.feather_ops.scaled_mm_any_m, registered in C++ with the native op
 # (csrc/torch_op.cpp): checks as validate_scaled_mm(block_divisible=False,
-# allow_bf16_a=True), the any_m_config tile, a Meta kernel for fake tensors.
+# allow_bf16_a=True), the any-M plan's tile and K split, a Meta kernel for fake tensors.
 _any_m_op = torch.ops.feather_ops.scaled_mm_any_m.default
 
 
@@ -317,7 +317,8 @@ def scaled_mm_hip_any_m(a, b_prepacked, scale, bias, out_dtype) -> torch.Tensor:
     kernels mask rows past M). Rows are independent, so the result equals
     padding M to a block multiple, calling scaled_mm_hip and slicing. `a` may
     also be bf16: it is then rounded to fp16 (round to nearest even) inside the
-    GEMM, the same values as calling it with a.to(torch.float16)."""
+    GEMM or by a cast pass before it, the same values as calling it with
+    a.to(torch.float16)."""
     return torch.ops.feather_ops.scaled_mm_any_m.default(a, b_prepacked, scale, bias, out_dtype)
 
 
@@ -325,8 +326,10 @@ def scaled_mm_hip_any_m_lora(a, b_prepacked, scale, bias, out_dtype, lora_t, lor
     """scaled_mm_hip_any_m(...) + lora_t @ lora_u.T: the unmerged-LoRA term
     (reference comfy_feather/lora.py:4-35) with the strengths folded into
     lora_t (M, R); lora_u is (N, R); both contiguous fp16 or bf16, R % 32 == 0.
-    On the large tiles the term joins the fp32 accumulator before the output
-    rounding (no second pass over C); other routes add it to C afterwards."""
+    Where any_m_config names a large LDS tile the term joins the fp32
+    accumulator before the output rounding; elsewhere it is added to the
+    finished result in the output type, in the epilogue of the kernels that
+    take it, else (e4m3fn weights, wide or split small-M strips) by a pass over C."""
     return torch.ops.feather_ops.scaled_mm_any_m_lora.default(a, b_prepacked, scale, bias, out_dtype, lora_t, lora_u)
 
 
