@@ -35,16 +35,45 @@
 
 namespace {
 
-at::Tensor& workspace_for(const at::Device& dev, hipStream_t stream, size_t nbytes) {
+// Scratch of at least nbytes for a call on `stream`, arrival counters (kCounterBytes at its
+// start) zero before the first use; every call leaves them zero. The eager calls of a stream
+// share one buffer, which is replaced when a call needs more. A call under stream capture never
+// gets that buffer (its address would stay in the graph after a replacement has freed it) and an
+// eager call none made under capture (its zero fill runs with the graph's replays only): the
+// calls of one capture on one stream share a buffer allocated and zeroed inside that capture,
+// whose memory torch keeps for the graph, so graphs share nothing with each other either. The
+// caller holds the returned tensor until its kernels are enqueued: a call of another thread on
+// this stream may replace the buffer meanwhile.
+at::Tensor workspace_for(const at::Device& dev, hipStream_t stream, size_t nbytes) {
+    constexpr int64_t kCounterBytes = 65536;
+    struct Buffers {
+        at::Tensor eager, captured;
+        unsigned long long capture = 0;
+    };
     static std::mutex mu;
-    static std::map<std::pair<int, hipStream_t>, at::Tensor> pool;
-    std::lock_guard<std::mutex> lock(mu);
-    at::Tensor& ws = pool[{dev.index(), stream}];
-    if (!ws.defined() || static_cast<size_t>(ws.numel()) < nbytes) {
-        const int64_t n = static_cast<int64_t>(nbytes > (size_t(1) << 20) ? nbytes : (size_t(1) << 20));
-        ws = at::zeros({n}, at::TensorOptions().dtype(at::kByte).device(dev));
+    static std::map<std::pair<int, hipStream_t>, Buffers> pool;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {
+        (void)hipGetLastError();  // (the legacy stream while another stream captures: not capturing itself)
+        status = hipStreamCaptureStatusNone;
     }
-    return ws;
+    const bool capturing = status == hipStreamCaptureStatusActive;
+    const int64_t n = static_cast<int64_t>(nbytes > (size_t(1) << 20) ? nbytes : (size_t(1) << 20));
+    const auto options = at::TensorOptions().dtype(at::kByte).device(dev);
+    std::lock_guard<std::mutex> lock(mu);
+    Buffers& b = pool[{dev.index(), stream}];
+    if (!capturing || b.capture != id) b.captured.reset();  // a capture that has ended: the graph's memory alone
+    if (!capturing) {
+        if (!b.eager.defined() || static_cast<size_t>(b.eager.numel()) < nbytes) b.eager = at::zeros({n}, options);
+        return b.eager;
+    }
+    b.capture = id;
+    if (!b.captured.defined() || static_cast<size_t>(b.captured.numel()) < nbytes) {
+        b.captured = at::empty({n}, options);
+        b.captured.narrow(0, 0, kCounterBytes).zero_();
+    }
+    return b.captured;
 }
 
 // Argument checks of the reference's scaled_mm (hip_kernel.cu:648-730).
@@ -125,8 +154,7 @@ struct Launch {
     int64_t M, N, K;
     int cfg[5];
     int b_dtype;
-    void* ws;
-    size_t ws_size;
+    at::Tensor ws;
     hipStream_t stream;
 
     bool operator()(const at::Tensor& a, int a_dtype) const {
@@ -135,8 +163,8 @@ struct Launch {
             scale.has_value() ? static_cast<const float*>(scale->data_ptr()) : nullptr,
             bias.has_value() ? static_cast<const uint16_t*>(bias->data_ptr()) : nullptr,
             static_cast<uint16_t*>(c.data_ptr()), M, N, K, scale.has_value() ? 1 : 0, bias.has_value() ? 1 : 0,
-            cfg[0], cfg[1], cfg[2], cfg[3], cfg[4], b_dtype, c.scalar_type() == at::kHalf ? 0 : 1, ws, ws_size,
-            stream);
+            cfg[0], cfg[1], cfg[2], cfg[3], cfg[4], b_dtype, c.scalar_type() == at::kHalf ? 0 : 1,
+            ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? static_cast<size_t>(ws.numel()) : 0, stream);
     }
 };
 
@@ -146,14 +174,10 @@ Launch make_launch(const at::Tensor& a, const at::Tensor& b_prepacked, const std
                    const std::optional<at::Tensor>& bias, const at::Tensor& c, const int (&cfg)[5], int b_dtype) {
     const hipStream_t stream = c10::hip::getCurrentHIPStream(a.device().index()).stream();
     const int64_t M = a.size(0), K = a.size(1), N = b_prepacked.size(1);
-    Launch l{b_prepacked, scale, bias, c, M, N, K, {cfg[0], cfg[1], cfg[2], cfg[3], cfg[4]}, b_dtype, nullptr, 0,
+    Launch l{b_prepacked, scale, bias, c, M, N, K, {cfg[0], cfg[1], cfg[2], cfg[3], cfg[4]}, b_dtype, at::Tensor(),
              stream};
     const size_t ws_bytes = feather_scaled_mm_workspace_size(M, N, K, cfg[0], cfg[1], cfg[2], cfg[3], cfg[4]);
-    if (ws_bytes) {
-        at::Tensor& t = workspace_for(a.device(), stream, ws_bytes);
-        l.ws = t.data_ptr();
-        l.ws_size = static_cast<size_t>(t.numel());
-    }
+    if (ws_bytes) l.ws = workspace_for(a.device(), stream, ws_bytes);
     return l;
 }
 
@@ -191,20 +215,15 @@ at::Tensor scaled_mm_any_m(const at::Tensor& a, const at::Tensor& b_prepacked, c
     check_args(a, b_prepacked, scale, bias, c, cfg[0], cfg[1], cfg[2], cfg[3], cfg[4], b_dtype, false, true);
     const hipStream_t stream = c10::hip::getCurrentHIPStream(a.device().index()).stream();
     auto launch = [&](const at::Tensor& x, int x_dtype) {
-        void* ws = nullptr;
-        size_t ws_size = 0;
         const size_t need = feather_scaled_mm_any_m_workspace_size(M, N, K);
-        if (need) {
-            at::Tensor& t = workspace_for(a.device(), stream, need);
-            ws = t.data_ptr();
-            ws_size = static_cast<size_t>(t.numel());
-        }
+        const at::Tensor ws = need ? workspace_for(a.device(), stream, need) : at::Tensor();
         return feather_launch_scaled_mm_any_m(
             x.data_ptr(), x_dtype, static_cast<const uint8_t*>(b_prepacked.data_ptr()),
             scale.has_value() ? static_cast<const float*>(scale->data_ptr()) : nullptr,
             bias.has_value() ? static_cast<const uint16_t*>(bias->data_ptr()) : nullptr,
             static_cast<uint16_t*>(c.data_ptr()), M, N, K, scale.has_value() ? 1 : 0, bias.has_value() ? 1 : 0,
-            b_dtype, out_dtype == at::kHalf ? 0 : 1, ws, ws_size, stream);
+            b_dtype, out_dtype == at::kHalf ? 0 : 1, need ? ws.data_ptr() : nullptr,
+            need ? static_cast<size_t>(ws.numel()) : 0, stream);
     };
     bool launched;
     if (a.scalar_type() == at::kBFloat16) {
@@ -281,14 +300,8 @@ at::Tensor scaled_mm_any_m_lora(const at::Tensor& a, const at::Tensor& b_prepack
     check_args(a, b_prepacked, scale, bias, c, cfg[0], cfg[1], cfg[2], cfg[3], cfg[4], b_dtype, false, true);
     const hipStream_t stream = c10::hip::getCurrentHIPStream(a.device().index()).stream();
     auto launch = [&](const at::Tensor& x, int x_dtype) {
-        void* ws = nullptr;
-        size_t ws_size = 0;
         const size_t need = feather_scaled_mm_any_m_lora_workspace_size(M, N, K);
-        if (need) {
-            at::Tensor& t = workspace_for(a.device(), stream, need);
-            ws = t.data_ptr();
-            ws_size = static_cast<size_t>(t.numel());
-        }
+        const at::Tensor ws = need ? workspace_for(a.device(), stream, need) : at::Tensor();
         return feather_launch_scaled_mm_any_m_lora(
             x.data_ptr(), x_dtype, static_cast<const uint8_t*>(b_prepacked.data_ptr()),
             scale.has_value() ? static_cast<const float*>(scale->data_ptr()) : nullptr,
@@ -296,7 +309,8 @@ at::Tensor scaled_mm_any_m_lora(const at::Tensor& a, const at::Tensor& b_prepack
             static_cast<uint16_t*>(c.data_ptr()), M, N, K, scale.has_value() ? 1 : 0, bias.has_value() ? 1 : 0,
             static_cast<const uint16_t*>(lora_t.data_ptr()), static_cast<const uint16_t*>(lora_u.data_ptr()), R,
             lora_t.scalar_type() == at::kHalf ? FEATHER_DTYPE_F16 : FEATHER_DTYPE_BF16, b_dtype,
-            out_dtype == at::kHalf ? 0 : 1, ws, ws_size, stream);
+            out_dtype == at::kHalf ? 0 : 1, need ? ws.data_ptr() : nullptr, need ? static_cast<size_t>(ws.numel()) : 0,
+            stream);
     };
     at::Tensor x = a;
     if (launch(a, a.scalar_type() == at::kHalf ? FEATHER_DTYPE_F16 : FEATHER_DTYPE_BF16)) return c;
@@ -336,7 +350,8 @@ at::Tensor lora_down(const at::Tensor& x, const at::Tensor& d) {
     const c10::DeviceGuard guard(x.device());
     const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
     const size_t ws_bytes = feather_lora_down_workspace_size(M, K, R);
-    void* ws = ws_bytes ? workspace_for(x.device(), stream, ws_bytes).data_ptr() : nullptr;
+    const at::Tensor wsbuf = ws_bytes ? workspace_for(x.device(), stream, ws_bytes) : at::Tensor();
+    void* ws = ws_bytes ? wsbuf.data_ptr() : nullptr;
     const int st = feather_lora_down(x.data_ptr(), x.scalar_type() == at::kHalf ? FEATHER_DTYPE_F16 : FEATHER_DTYPE_BF16,
                                      d.data_ptr(), t.data_ptr(), M, K, R, ws, ws_bytes, stream);
     TORCH_CHECK(st == FEATHER_OK, "feather_lora_down failed: ", feather_status_string(st));
@@ -359,7 +374,8 @@ std::tuple<at::Tensor, at::Tensor> lora_down_cast(const at::Tensor& x, const at:
     const c10::DeviceGuard guard(x.device());
     const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
     const size_t ws_bytes = feather_lora_down_workspace_size(M, K, R);
-    void* ws = ws_bytes ? workspace_for(x.device(), stream, ws_bytes).data_ptr() : nullptr;
+    const at::Tensor wsbuf = ws_bytes ? workspace_for(x.device(), stream, ws_bytes) : at::Tensor();
+    void* ws = ws_bytes ? wsbuf.data_ptr() : nullptr;
     const int st = feather_lora_down_cast(x.data_ptr(), d.data_ptr(), t.data_ptr(), static_cast<uint16_t*>(x16.data_ptr()),
                                           M, K, R, ws, ws_bytes, stream);
     TORCH_CHECK(st == FEATHER_OK, "feather_lora_down_cast failed: ", feather_status_string(st));
@@ -411,7 +427,7 @@ std::tuple<at::Tensor, at::Tensor> quantize_prepack_e5m2(const at::Tensor& w, co
     const hipStream_t stream = c10::hip::getCurrentHIPStream(src.device().index()).stream();
     // the stream's zero-filled workspace (its counter region is left zero)
     const size_t ws_bytes = feather_quantize_workspace_size();
-    at::Tensor& ws = workspace_for(src.device(), stream, ws_bytes);
+    const at::Tensor ws = workspace_for(src.device(), stream, ws_bytes);
     const int st = feather_quantize_prepack_e5m2_ws(src.data_ptr(), code, N, K,
                                                     cs.defined() ? static_cast<const float*>(cs.data_ptr()) : nullptr,
                                                     native ? 1 : 0, static_cast<uint8_t*>(out.data_ptr()),
