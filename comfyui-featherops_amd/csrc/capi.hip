@@ -305,6 +305,13 @@ int feather_scaled_mm_any_m_plan(int64_t M, int64_t N, int64_t K, int* ksplit) {
     return pl.tile;
 }
 
+int feather_scaled_mm_any_m_smallm_form(int64_t M, int64_t N, int64_t K, int lora) {
+    if (M <= 0 || !sizes_ok(M, N, K)) return 0;
+    const int cus = plan_cus();
+    const feather::MmPlan pl = lora ? feather::plan_scaled_mm_lora(M, N, K, cus) : feather::plan_scaled_mm(M, N, K, cus);
+    return pl.tile == feather::kSmallM ? feather::smallm_form(M, N, K, cus, pl.strip, pl.ksplit) : 0;
+}
+
 bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b_prepacked, const float* scale,
                                     const uint16_t* bias, uint16_t* c, int64_t M, int64_t N, int64_t K, int has_scale,
                                     int has_bias, int b_dtype, int output_dtype, void* workspace,
@@ -329,7 +336,7 @@ bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b
     const bool room = workspace != nullptr && workspace_bytes >= pl.workspace_bytes;
     if (pl.tile == feather::kSmallM)
         return feather::launch_smallm_kernel(p, pl.ksplit > 1 && room ? workspace : nullptr,
-                                             pl.ksplit > 1 && room ? workspace_bytes : 0, stream);
+                                             pl.ksplit > 1 && room ? workspace_bytes : 0, stream, pl.strip, pl.ksplit);
     return feather::launch_tile(pl.tile, p, room ? pl.ksplit : 1, workspace, workspace_bytes, stream);
 }
 
@@ -370,7 +377,7 @@ bool feather_launch_scaled_mm_any_m_lora(const void* a, int a_dtype, const uint8
                                     nullptr, 0, stream);
     const feather::MmPlan pl = feather::plan_scaled_mm_lora(M, N, K, plan_cus());
     const bool room = workspace != nullptr && workspace_bytes >= pl.workspace_bytes;
-    if (pl.tile == feather::kSmallM) return p.lora_after && feather::launch_smallm_kernel(p, nullptr, 0, stream);
+    if (pl.tile == feather::kSmallM) return p.lora_after && feather::launch_smallm_kernel(p, nullptr, 0, stream, pl.strip, pl.ksplit);
     const bool large = pl.tile >= feather::kLds256x256 && pl.tile < feather::kLdsSk64x64;
     if (large && p.lora_after) return false;
     // the 128 x 384 tile's stage buffers cannot hold 64 ranks of its U rows

@@ -78,9 +78,13 @@ constexpr size_t kWorkspaceCounterBytes = static_cast<size_t>(kWorkspaceCounters
 // Small-M kernel. With a workspace of at least smallm_workspace_bytes() it
 // also splits K across workgroups; without one it splits K inside each
 // workgroup only.
-bool launch_smallm_kernel(const MmArgs& p, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// strip: column tiles per strip and ksplit workgroups per strip as a plan chose them; 0: by the
+// kernel's own cost model. Without the workspace a split needs, K is split inside the workgroup only.
+bool launch_smallm_kernel(const MmArgs& p, void* workspace, size_t workspace_bytes, hipStream_t stream, int strip = 0,
+                          int ksplit = 0);
 size_t smallm_workspace_bytes(int64_t M, int64_t N, int64_t K, int target_groups);
 int smallm_ksplit(int64_t M, int64_t N, int64_t K, int target_groups);
+size_t smallm_split_bytes(int64_t M, int64_t N, int strip, int ksplit);
 bool launch_lds_kernel(int kernel_id, const MmArgs& p, hipStream_t stream);
 
 struct SplitKPlan {
@@ -92,19 +96,24 @@ struct SplitKPlan {
 };
 SplitKPlan lds_splitk_plan(int64_t M, int64_t N, int64_t K, int target);
 
-// What serves one call: a KernelId and the K split across workgroups (small-M:
-// ksplit > 1 allows that kernel's own split).
+// What serves one call: a KernelId, the K split across workgroups and, for the small-M kernel,
+// the column tiles per strip (0: that kernel's own choice of both).
 struct MmPlan {
     int tile = kKernelNone;
     int ksplit = 1;
     size_t workspace_bytes = 0;
+    int strip = 0;
 };
 // The variant with the least modelled time (scaled_mm_plan.hip): the same for every
 // type, so bf16 activations give the bits of their fp16 cast.
 MmPlan plan_scaled_mm(int64_t M, int64_t N, int64_t K, int cus);
 // The same for a call with a rank-R term: the small-M kernel only where its lean form, which adds it, serves the shape.
 MmPlan plan_scaled_mm_lora(int64_t M, int64_t N, int64_t K, int cus);
-bool smallm_is_lean(int64_t M, int64_t N, int64_t K, int target_groups, bool allow_split);
+// The kernel behind a small-M launch: the general kernel on 16-column strips or wider ones, or
+// the lean kernel with one workgroup per CU or two.
+enum SmallmForm : int { kSmallmStrips = 1, kSmallmWide = 2, kSmallmLean = 3, kSmallmLeanPair = 4 };
+SmallmForm smallm_form(int64_t M, int64_t N, int64_t K, int target_groups, int strip, int ksplit);
+inline bool is_lean(SmallmForm f) { return f == kSmallmLean || f == kSmallmLeanPair; }
 // Counter region + fp32 partial tiles of a K split (0 for ksplit 1).
 size_t tile_workspace_bytes(int tile, int64_t M, int64_t N, int ksplit);
 // Launches a tile with the given K split; ksplit > 1 needs tile_workspace_bytes() of

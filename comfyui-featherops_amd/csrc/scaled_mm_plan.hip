@@ -64,23 +64,61 @@ double cost_us(const TileCost& t, int64_t tiles, int64_t stages, int ks, int cus
     return us;
 }
 
-// Small-M kernel, 17..48 rows. Up to 32: the lean kernel on unsplit 16-column strips
-// (K % 64 == 0: fit of 29 shapes, 3.5% rms; otherwise the general kernel on those strips,
-// of 23 shapes, 11% rms; the split plans lose to the 32-row tiles: M=22 N=1152
-// K=10304 12.0 vs 8.6 us, M=19 N=8576 K=6144 15.3 vs 11.8). 33..48 rows: unsplit
-// strips with K < 2048 (M=34 N=1792 K=1392 4.8 vs 5.4 us; longer K: M=38 N=2176
-// K=6848 14.8 vs 9.1).
-double smallm_us(int64_t M, int64_t N, int64_t K, int cus) {
-    const double mb = static_cast<double>(N) * static_cast<double>(K) * 1e-6;
-    const double rounds = static_cast<double>(ceil_div(ceil_div(N, 16), cus));
-    const double steps = rounds * static_cast<double>(ceil_div(K, 64));
-    if (M <= 32 && K % 64 == 0)
-        return 1.78 + 0.706 * static_cast<double>(ceil_div(N, 16)) / cus + (0.0178 + 0.0012 * static_cast<double>(M)) * steps +
-               0.0095 * mb;
-    if (M <= 32) return 2.16 + 0.13 * rounds + (0.0347 + 0.0011 * static_cast<double>(M - 17)) * steps + 0.071 * mb;
-    if (M <= 48 && K < 2048)
-        return 1.02 + 0.63 * rounds + (0.108 + 0.0017 * static_cast<double>(M - 33)) * steps + 0.40 * mb;
-    return 1e30;
+// Small-M kernel, 17..48 rows: its form with the least modelled time, from graph-replayed runs
+// that rotate weights past the MALL (a model's layers find their weights in HBM; fits of weights
+// that stay in the MALL are up to 40% low on these forms). tile_us: the best tile, the same way.
+// A form whose launch takes bf16 activations spares them the cast pass that every tile needs
+// (2.3-2.9 us), and both activation types take one plan: such a form may be slower than the tile by
+// that much unsplit, and by less where the tile's gain on fp16 calls is larger than the cast's
+// cost to bf16 ones (K splits, weights above 4096 x 4096; none past one round of strips of those).
+// strip 0: the tile.
+struct SmallmChoice {
+    int strip = 0, ksplit = 1;
+};
+
+SmallmChoice smallm_choice(int64_t M, int64_t N, int64_t K, int cus, bool lora, double tile_us) {
+    const int64_t stages = ceil_div(K, 64), strips = ceil_div(N, 16);
+    const double m = static_cast<double>(M), nst = static_cast<double>(stages);
+    const double mb = static_cast<double>(N) * static_cast<double>(K) * 1e-6, a = m * static_cast<double>(K) * 1e-6;
+    if (M > 32) {
+        // unsplit 16-column strips, one workgroup per CU, which read fp16 activations; rows whose
+        // pitch is a multiple of 128 bytes read slower (59 shapes, 3% rms). From K = 2048 on a
+        // tile wins (M=34 N=736 K=9744 18.6 vs 8.6 us), past one round too (M=40 N=5456 K=320 6.2 vs 4.4)
+        const double us = K % 64 == 0 ? 2.78 + 0.0033 * m * nst + 0.213 * mb : 2.56 + (0.049 + 0.0012 * m) * nst + 0.14 * mb;
+        return {K < 2048 && strips <= cus && !lora && us <= tile_us ? 1 : 0, 1};
+    }
+    const bool large = N * K > int64_t(4096) * 4096;
+    const double slack = !large ? 2.5 : strips <= cus ? 2.0 : 0.0;
+    SmallmChoice best;
+    double best_us = 1e30;
+    bool take = false;
+    auto offer = [&](int ks, double us, double allowed) {
+        take = take || us <= tile_us + allowed;
+        if (us < best_us) best_us = us, best = {1, ks};
+    };
+    if (K % 64 == 0) {
+        // the lean kernel, two workgroups per CU (134 shapes, 6.3% rms); a short K on more than two
+        // rounds of strips is the tiles' (M=26 N=13696 K=384 5.5 vs 4.5 us)
+        const double rounds = static_cast<double>(ceil_div(strips, cus));
+        if ((strips <= 2 * cus || K >= 512) && (!lora || is_lean(smallm_form(M, N, K, cus, 1, 1))))
+            offer(1, 1.89 + 0.484 * rounds + (0.0017 + 0.0011 * m + 0.085 * a) * rounds * nst + 0.156 * mb, slack);
+    } else if (strips <= cus) {
+        // the general kernel on 16-column strips (105 shapes, 6% rms)
+        if (!lora) offer(1, 2.82 + (0.015 + 0.0009 * m + 0.087 * a) * nst + 0.212 * mb, slack);
+    } else if (K < 1600 && !lora) {
+        // past one round of those, 64-column strips (fp16 activations): 2-9% less than the best tile on 8
+        // of 9 shapes up to K = 1504 (M=23 N=9520 K=752 4.8 vs 5.1 us), 1-4% more from K = 2208 on;
+        // 16-column strips M=32 N=8432 K=1104 11.1 vs 6.8
+        return {4, 1};
+    }
+    // K split of 16-column strips in one round (81 shapes, 3.9% rms, and 0.3 us that it has to be worth):
+    // long K on narrow weights (M=31 N=640 K=9696 12.2 us unsplit, 7.9 in four splits). Wide split strips
+    // lose to the 32-row tiles
+    if (!lora)
+        for (int ks = 2; ks <= 8 && ks * 16 <= stages && ks * strips <= cus; ++ks)
+            offer(ks, 3.85 + (0.0187 + 0.0015 * m) * static_cast<double>(ceil_div(stages, ks)) + 0.393 * ks + 0.15 * mb,
+                  0.4 * slack);
+    return take ? best : SmallmChoice{};
 }
 
 const TileCost* tile_cost(int tile) {
@@ -91,8 +129,7 @@ const TileCost* tile_cost(int tile) {
 
 MmPlan make_plan(int64_t M, int64_t N, int64_t K, int cus, bool lora) {
     MmPlan best;
-    const bool lean = M <= 32 && smallm_is_lean(M, N, K, cus, M <= 16);
-    if (M <= 16 && (!lora || lean)) {
+    if (M <= 16 && (!lora || is_lean(smallm_form(M, N, K, cus, 0, 0)))) {
         // one row tile: the small-M kernel and its own plan. The 32 x 64 tile took up to 8%
         // less on a few wide weights (M=16 N=13824 K=5120 13.2 vs 14.3 us), but bf16
         // activations would need a cast pass of 3.5 us first, and both types take one plan
@@ -128,13 +165,11 @@ MmPlan make_plan(int64_t M, int64_t N, int64_t K, int cus, bool lora) {
         }
     }
     best.workspace_bytes = tile_workspace_bytes(best.tile, M, N, best.ksplit);
-    if (M > 16 && M <= 48 && (!lora || lean)) {
-        // bf16 activations cost a cast pass (3.5 us and more) before a tile, none on the
-        // small-M kernel, and both types take one plan: where a weight is too small to
-        // make the tiles the better choice for most rows, they have to win by that much
-        const bool large = N * K > int64_t(4096) * 4096;
-        const double margin = !large && (M <= 32 || N < 3072) ? 3.5 : 0.0;
-        if (smallm_us(M, N, K, cus) <= best_us + margin) best = MmPlan{kSmallM, 1, 0};
+    if (M > 16 && M <= 48) {
+        // the table's time with the weight in HBM (190 shapes of 17..48 rows, 4.4% rms)
+        const double tile_us = 0.94 * best_us + 0.1e-6 * static_cast<double>(N) * static_cast<double>(K);
+        const SmallmChoice c = smallm_choice(M, N, K, cus, lora, tile_us);
+        if (c.strip > 0) best = MmPlan{kSmallM, c.ksplit, smallm_split_bytes(M, N, c.strip, c.ksplit), c.strip};
     }
     return best;
 }

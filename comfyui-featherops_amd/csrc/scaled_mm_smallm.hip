@@ -266,8 +266,10 @@ __global__ __launch_bounds__(64 * kWaves) void scaled_mm_smallm_kernel(
 // 8.0. With one workgroup per CU at most, the deeper form streams as fast or
 // faster (M=16 N=K=4096 5.16 vs 6.03 us, M=13 N=3520 K=4096 4.86 vs 5.84; short K
 // the other way by under 4%), so one row tile takes it there. Two row tiles are
-// always this form (M=20 N=K=4096 6.0 -> 5.6 us, M=18 N=3712 K=11392 10.7 -> 9.5,
-// M=24 N=8192 K=2048 7.1 -> 6.3; at most 3% slower, M=30 N=1792 K=2112 3.76 vs 3.87).
+// always this form: with the weight in HBM M=18 N=720 K=6144 7.3 -> 5.8 us, M=25 N=592
+// K=3904 5.5 -> 5.1, M=29 N=3120 K=3072 6.8 -> 6.7, and up to 6% slower on short K (M=18
+// N=848 K=1088 3.04 vs 3.21); against 64-column strips of the general kernel M=24 N=8192
+// K=2048 8.5 -> 7.4 (bf16 activations, which those do not take, 11.0 -> 7.8).
 // kLora: adds the rank-R term T . U^T (T (M, R), U (N, R), fp16 or bf16 by lora_bf16,
 // R % 32 == 0) to the finished result in the output type: wave t multiplies row tile
 // t's 16 x 16 product (fp32 MFMA sums, rounded to the factors' type and to the output
@@ -606,13 +608,18 @@ int smallm_ksplit(int64_t M, int64_t N, int64_t K, int target_groups) {
     return smallm_plan(M, N, K, target_groups).ks;
 }
 
-size_t smallm_workspace_bytes(int64_t M, int64_t N, int64_t K, int target_groups) {
-    const SmallmPlan pl = smallm_plan(M, N, K, target_groups);
+// The fixed counter region, then a partial tile per split and strip (0 unsplit).
+static size_t split_bytes(int64_t M, int64_t N, const SmallmPlan& pl) {
     if (pl.ks <= 1) return 0;
     const int64_t nstrips = (N + 16 * pl.ct - 1) / (16 * pl.ct);
-    // the fixed counter region, then ksplit partial tiles per strip
     return kWorkspaceCounterBytes + static_cast<size_t>(nstrips) * pl.ks * M * 16 * pl.ct * 4;
 }
+
+size_t smallm_workspace_bytes(int64_t M, int64_t N, int64_t K, int target_groups) {
+    return split_bytes(M, N, smallm_plan(M, N, K, target_groups));
+}
+
+size_t smallm_split_bytes(int64_t M, int64_t N, int strip, int ksplit) { return split_bytes(M, N, {strip, ksplit}); }
 
 // FEATHEROPS_SMALLM_LEAN=0 routes M <= 16 calls to the general small-M kernel
 // instead of the lean one (read once; for A/B timing).
@@ -624,22 +631,29 @@ static bool m16_disabled() {
     return off;
 }
 
-bool smallm_is_lean(int64_t M, int64_t N, int64_t K, int target_groups, bool allow_split) {
-    if (M <= 0 || M > 32) return false;
-    const SmallmPlan pl = smallm_plan(M, N, K, target_groups, allow_split);
-    return pl.ks == 1 && pl.ct == 1 && M * K * 2 < (int64_t(1) << 32) && K % 64 == 0 && N % 16 == 0 && !m16_disabled();
+static SmallmForm form_of(int64_t M, int64_t N, int64_t K, int cus, const SmallmPlan& pl) {
+    if (M <= 32 && pl.ks == 1 && pl.ct == 1 && M * K * 2 < (int64_t(1) << 32) && K % 64 == 0 && N % 16 == 0 &&
+        !m16_disabled())
+        return M > 16 || N / 16 > cus ? kSmallmLeanPair : kSmallmLean;
+    return pl.ct >= 2 ? kSmallmWide : kSmallmStrips;
 }
 
-bool launch_smallm_kernel(const MmArgs& p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+SmallmForm smallm_form(int64_t M, int64_t N, int64_t K, int target_groups, int strip, int ksplit) {
+    return form_of(M, N, K, target_groups > 0 ? target_groups : 256,
+                   strip > 0 ? SmallmPlan{strip, ksplit} : smallm_plan(M, N, K, target_groups));
+}
+
+bool launch_smallm_kernel(const MmArgs& p, void* workspace, size_t workspace_bytes, hipStream_t stream, int strip,
+                          int ksplit) {
     if (p.M <= 0 || p.M > 64) return false;
     const int mt = mt_of(p.M);
     const int target = p.smallm_min_groups > 0 ? p.smallm_min_groups : 256;
-    SmallmPlan pl = smallm_plan(p.M, p.N, p.K, target);
+    SmallmPlan pl = strip > 0 ? SmallmPlan{strip, ksplit} : smallm_plan(p.M, p.N, p.K, target);
     float* partials = nullptr;
     uint32_t* counters = nullptr;
-    if (pl.ks > 1 && (workspace == nullptr || workspace_bytes < smallm_workspace_bytes(p.M, p.N, p.K, target))) {
+    if (pl.ks > 1 && (workspace == nullptr || workspace_bytes < split_bytes(p.M, p.N, pl))) {
         // no (or too small a) workspace: split K inside each workgroup only
-        pl = smallm_plan(p.M, p.N, p.K, target, false);
+        pl = strip > 0 ? SmallmPlan{strip, 1} : smallm_plan(p.M, p.N, p.K, target, false);
     }
     if (pl.ks > 1) {
         counters = static_cast<uint32_t*>(workspace);
@@ -649,9 +663,10 @@ bool launch_smallm_kernel(const MmArgs& p, void* workspace, size_t workspace_byt
     const bool wide = pl.ct >= 2;
     // A through LDS needs every byte offset into A to fit the copy's 32-bit lane offset
     const bool lds_a = p.M * p.K * 2 < (int64_t(1) << 32);
-    if (mt <= 2 && ks == 1 && !wide && lds_a && p.K % 64 == 0 && p.N % 16 == 0 && !m16_disabled()) {
+    const SmallmForm form = form_of(p.M, p.N, p.K, target, pl);
+    if (is_lean(form)) {
         if (mt == 2) return launch_m16<2, true>(p, stream);
-        return p.N / 16 > target ? launch_m16<1, true>(p, stream) : launch_m16<1, false>(p, stream);
+        return form == kSmallmLeanPair ? launch_m16<1, true>(p, stream) : launch_m16<1, false>(p, stream);
     }
     if (p.lora_dtype != 0) return false;  // only the lean kernel adds a rank-R term
     switch (mt) {

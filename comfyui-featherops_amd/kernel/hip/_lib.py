@@ -35,6 +35,7 @@ SIGNATURES: dict[str, tuple] = {
     "feather_launch_scaled_mm_any_m": (ctypes.c_bool, [_vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _int,
                                                        _int, _int, _vp, ctypes.c_size_t, _vp]),
     "feather_scaled_mm_any_m_plan": (_int, [_i64, _i64, _i64, ctypes.POINTER(ctypes.c_int)]),
+    "feather_scaled_mm_any_m_smallm_form": (_int, [_i64, _i64, _i64, _int]),
     "feather_scaled_mm_any_m_workspace_size": (ctypes.c_size_t, [_i64, _i64, _i64]),
     "feather_scaled_mm_any_m_lora_workspace_size": (ctypes.c_size_t, [_i64, _i64, _i64]),
     "feather_launch_scaled_mm_any_m_lora": (ctypes.c_bool, [_vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int,

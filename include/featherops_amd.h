@@ -120,6 +120,10 @@ bool feather_launch_scaled_mm_ex(const void* a, int a_dtype, const uint8_t* b_pr
 size_t feather_scaled_mm_any_m_workspace_size(int64_t M, int64_t N, int64_t K);
 /* The kernel id (csrc/scaled_mm_dispatch.h) that entry takes and, in *ksplit (may be NULL), its K split. */
 int feather_scaled_mm_any_m_plan(int64_t M, int64_t N, int64_t K, int* ksplit);
+/* The form of the small-M kernel it takes (lora: the entry with a rank-R term below): 0 another kernel, 1 16-column
+ * strips, 2 wider strips, 3 the lean kernel, 4 the lean kernel with two workgroups per CU. Up to 32 rows, forms 1, 3
+ * and 4 take bf16 activations. */
+int feather_scaled_mm_any_m_smallm_form(int64_t M, int64_t N, int64_t K, int lora);
 bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b_prepacked, const float* scale,
                                     const uint16_t* bias, uint16_t* c, int64_t M, int64_t N, int64_t K, int has_scale,
                                     int has_bias, int b_dtype, int output_dtype, void* workspace,

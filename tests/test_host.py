@@ -396,3 +396,60 @@ def test_any_m_plan_is_launchable(pkg):
     assert seen == {10} | set(two_groups) | one_group
     assert L.feather_scaled_mm_any_m_plan(16, 24, 64, None) == 0  # N % 16 != 0
     assert not L.feather_launch_scaled_mm_any_m(None, 0, None, None, None, None, 16, 24, 64, 0, 0, 1, 0, None, 0, None)
+
+
+def _any_m_plan(L, M, N, K):
+    import ctypes
+
+    ks = ctypes.c_int(-1)
+    kid = L.feather_scaled_mm_any_m_plan(M, N, K, ctypes.byref(ks))
+    return kid, ks.value, L.feather_scaled_mm_any_m_smallm_form(M, N, K, 0)
+
+
+def test_small_m_plan_and_launch_share_one_form(pkg):
+    """The small-M kernel's form that the any-M plan prices is the one its launch takes: unsplit 17..32 rows
+    with K % 64 == 0 run the lean kernel, two workgroups per CU, at any width; a rank-R term runs on it
+    alone; a K split fits one round and leaves no split without a stage per wave."""
+    import random
+
+    from featherops_amd.kernel.hip import _lib
+
+    L = _lib.lib()
+    rng = random.Random(9)
+    seen = set()
+    for _ in range(20000):
+        M, N, K = rng.randint(17, 48), 16 * int(2 ** rng.uniform(2, 10)), 16 * int(2 ** rng.uniform(0, 10))
+        kid, ks, form = _any_m_plan(L, M, N, K)
+        lora = L.feather_scaled_mm_any_m_smallm_form(M, N, K, 1)
+        assert lora in (0, 4) and (lora == 0 or M <= 32), (M, N, K, lora)
+        assert (kid == 10) == (form != 0), (M, N, K, kid, form)
+        if kid != 10:
+            continue
+        seen.add((M <= 32, form, ks > 1))
+        if M <= 32 and K % 64 == 0 and ks == 1:
+            assert form == 4, (M, N, K, form)
+        if ks > 1:
+            assert M <= 32 and N // 16 * ks <= 256 and -(-K // 64) >= 16 * ks
+            nbytes = L.feather_scaled_mm_any_m_workspace_size(M, N, K)
+            assert nbytes == 65536 + N // 16 * ks * M * 16 * 4
+    assert seen == {(True, 4, False), (True, 1, False), (True, 1, True), (True, 2, False), (False, 1, False)}, seen
+
+
+@pytest.mark.parametrize("M,N,K,small_m,split", [
+    # us on cold weights, small-M form and best tile: kernel that the plan has to take
+    (31, 640, 9696, True, True),    # four K splits 7.9 (bf16 8.2), unsplit 12.2, tile 7.9 (bf16 10.8)
+    (23, 832, 10864, True, True),   # 8.9 (bf16 9.3), unsplit 17.3, tile 9.1 (bf16 11.8)
+    (26, 944, 10944, True, True),   # 9.0 (bf16 9.4), unsplit 14.2, tile 9.3 (bf16 12.0)
+    (24, 4480, 3328, True, False),  # lean 10.0 (bf16 10.4), wide strips 11.7, tile 8.1 (bf16 11)
+    (30, 7488, 1024, True, False),  # lean 4.6 (bf16 5.1), wide strips 5.9 (bf16 8.1), tile 5.2 (bf16 7.4)
+    (30, 4992, 3152, False, False),  # wide strips 12.8, tile 8.7
+    (48, 2976, 2016, False, False),  # 16-column strips 6.8 (bf16 9.1), tile 6.5 (bf16 8.9)
+    (47, 1488, 1792, False, False),  # 7.7 (bf16 10.0), tile 5.9 (bf16 8.4)
+    (40, 5456, 320, False, False),   # 6.2 (bf16 8.4), tile 4.4 (bf16 6.6)
+])
+def test_small_m_plan_on_measured_shapes(pkg, M, N, K, small_m, split):
+    from featherops_amd.kernel.hip import _lib
+
+    kid, ks, form = _any_m_plan(_lib.lib(), M, N, K)
+    assert (kid == 10) == small_m, (kid, ks, form)
+    assert not small_m or (ks > 1) == split, (kid, ks, form)
