@@ -1,6 +1,7 @@
 """The lean small-M kernel with two workgroups per CU (M <= 16 and more 16-column strips than CUs;
-every M of 17..32): whole outputs against a float64 evaluation on the device, and the bits of the
-same columns from a call of at most one strip per CU (both forms add in one order)."""
+17..32 rows, at any width): whole outputs against a float64 evaluation on the device, and the bits of
+the same columns from a call of at most one strip per CU (both forms add in one order). Every case
+asks the plan that this kernel serves it."""
 
 import ctypes
 
@@ -12,9 +13,17 @@ from gpu_util import assert_gemm_close_dev, lib, torch_ref_dev
 pytestmark = pytest.mark.gpu
 
 # M at the edges of 8-row copies and 16-row tiles; one strip past the CU count, a partial and a full
-# second round, a third; K below one stage per wave, one past a round of stages (16 waves x 2), long
-CASES = [(1, 4112, 64), (1, 12288, 3072), (8, 8208, 1088), (9, 8192, 2112), (16, 4144, 4096), (3, 12304, 2048),
-         (17, 1040, 64), (24, 4096, 1088), (32, 4112, 2112), (25, 8192, 1024)]
+# second round, a third (769 strips); K below one stage per wave, one past a round of
+# stages (16 waves x 2; two row tiles 16 x 1), long
+CASES = [(1, 4112, 64), (1, 12288, 3072), (8, 8208, 640), (9, 8192, 2112), (16, 4144, 2112), (3, 12304, 64),
+         (17, 1040, 64), (24, 4096, 1088), (32, 4112, 2112), (25, 8192, 1024), (18, 8208, 576), (30, 12304, 1088)]
+LEAN, LEAN_PAIR = 3, 4
+
+
+def _form(M, N, K, lora=0):
+    ks = ctypes.c_int()
+    assert lib().feather_scaled_mm_any_m_plan(M, N, K, ctypes.byref(ks)) == 10 and ks.value == 1
+    return lib().feather_scaled_mm_any_m_smallm_form(M, N, K, lora)
 
 
 @pytest.mark.parametrize("a_dtype,b_dtype,out_dtype", [
@@ -23,8 +32,7 @@ CASES = [(1, 4112, 64), (1, 12288, 3072), (8, 8208, 1088), (9, 8192, 2112), (16,
 @pytest.mark.parametrize("M,N,K", CASES)
 def test_small_m_pair(cuda, hk, M, N, K, a_dtype, b_dtype, out_dtype):
     e4m3 = b_dtype == torch.float8_e4m3fn
-    ks = ctypes.c_int()
-    assert lib().feather_scaled_mm_any_m_plan(M, N, K, ctypes.byref(ks)) == 10 and ks.value == 1
+    assert _form(M, N, K) == LEAN_PAIR
     print("small-M pair", M, N, K, a_dtype, b_dtype, out_dtype, flush=True)
     g = torch.Generator(device=cuda).manual_seed(M + N + K)
     a = torch.randn(M, K, generator=g, device=cuda).to(a_dtype)
@@ -38,17 +46,16 @@ def test_small_m_pair(cuda, hk, M, N, K, a_dtype, b_dtype, out_dtype):
     n1 = 2048 if M <= 16 else 1024
     for n0 in range(0, N, n1):
         part = bp[:, n0:n0 + n1].contiguous()
-        if lib().feather_scaled_mm_any_m_plan(M, part.shape[1], K, ctypes.byref(ks)) == 10 and ks.value == 1:
-            yp = hk.scaled_mm_hip_any_m(a, part, s, bias[n0:n0 + n1].contiguous(), out_dtype)
-            assert torch.equal(yp.view(torch.int16), y[:, n0:n0 + n1].contiguous().view(torch.int16)), n0
+        assert _form(M, part.shape[1], K) == (LEAN if M <= 16 else LEAN_PAIR)
+        yp = hk.scaled_mm_hip_any_m(a, part, s, bias[n0:n0 + n1].contiguous(), out_dtype)
+        assert torch.equal(yp.view(torch.int16), y[:, n0:n0 + n1].contiguous().view(torch.int16)), n0
 
 
-@pytest.mark.parametrize("M,N,K,R", [(1, 4112, 1088, 32), (16, 8192, 2112, 64), (20, 4112, 64, 32)])
+@pytest.mark.parametrize("M,N,K,R", [(1, 4112, 1088, 32), (16, 8192, 2112, 64), (20, 4112, 64, 32), (32, 8208, 1088, 160)])
 def test_small_m_pair_lora(cuda, hk, M, N, K, R):
     """The rank-R term is added to the finished result in the output type: the bits of the plain call
     plus the rounded product, up to the term's own rounding to the factors' type (fp32 sums of R terms)."""
-    ks = ctypes.c_int()
-    assert lib().feather_scaled_mm_any_m_plan(M, N, K, ctypes.byref(ks)) == 10 and ks.value == 1
+    assert _form(M, N, K) == LEAN_PAIR and _form(M, N, K, lora=1) == LEAN_PAIR
     print("small-M pair lora", M, N, K, R, flush=True)
     g = torch.Generator(device=cuda).manual_seed(M + N + K)
     a = torch.randn(M, K, generator=g, device=cuda).bfloat16()
