@@ -549,16 +549,19 @@ double smallm_cost_us(int64_t M, int64_t N, int64_t K, int ct, int ks, int cus) 
         // one row tile: least-squares fits of measured back-to-back times
         // (M = 1..16, N = 2048..13824, K = 5120..16384), one per kernel: the
         // lean kernel (16-column strips, no split) with one workgroup per CU
-        // and with two (46 shapes of more strips than CUs; its rounds hold twice
-        // as many), the general kernel with 16-column strips split over K, and
-        // 64-column strips, unsplit and split over K. Of the 46 shapes the choice
-        // costs 0.5% over the best of each, 5% at most (M=16 N=12288 K=3072 9.9 on
-        // wide strips, 9.4 as a pair; M=16 N=13824 K=5120 14.3 and 16.2)
+        // and with two (its rounds hold twice as many), the general kernel with
+        // 16-column strips split over K, and 64-column strips, unsplit and split
+        // over K. All on weights from HBM; the pair and the unsplit 64-column
+        // strips on 63 shapes of more strips than CUs (4.4% and 4.9% rms). Fitted to
+        // weights that stay in the MALL these two were 20% low beside the split forms
+        // (M=16 N=5600 K=6848: 15.5 us as a pair, 12.9 in two splits of 64-column
+        // strips). Of the 63 shapes the choice costs 0.4% over the best of each, 8% at most (M=13
+        // N=9680 K=640 4.6 on wide strips, 4.3 as a pair)
         struct Fit { double c0, round, kb, kb_row, mb; };
         constexpr Fit kLean{0.05, 1.80, 0.0213, 0.0012, 0.086};
-        constexpr Fit kLeanPair{1.12, 0.83, 0.0080, 0.0013, 0.0881};
+        constexpr Fit kLeanPair{1.53, 0.606, 0.0265, 0.0013, 0.0671};
         constexpr Fit kStripSplit{1.51, 2.70, 0.0184, 0.0009, 0.122};
-        constexpr Fit kWide{0.0, 3.0, 0.0064, 0.0003, 0.100};
+        constexpr Fit kWide{0.0, 2.94, 0.0165, 0.0004, 0.095};
         constexpr Fit kWideSplit{2.57, 2.99, 0.0108, 0.0003, 0.116};
         const bool pair = ct == 1 && ks == 1 && groups > cus && K % 64 == 0;
         const Fit& f = ct >= 4 ? (ks > 1 ? kWideSplit : kWide) : ks > 1 ? kStripSplit : pair ? kLeanPair : kLean;

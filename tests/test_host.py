@@ -453,3 +453,18 @@ def test_small_m_plan_on_measured_shapes(pkg, M, N, K, small_m, split):
     kid, ks, form = _any_m_plan(_lib.lib(), M, N, K)
     assert (kid == 10) == small_m, (kid, ks, form)
     assert not small_m or (ks > 1) == split, (kid, ks, form)
+
+
+@pytest.mark.parametrize("M,N,K,form,ksplit", [
+    # us on cold weights: the lean kernel with two workgroups per CU and the best form of 64-column strips
+    (16, 5600, 6848, 2, 2),   # 15.5, two splits 12.9
+    (8, 4864, 8896, 2, 3),    # 15.4, three splits 13.0
+    (11, 5104, 10880, 2, 3),  # 19.8, three splits 15.1
+    (2, 8640, 5440, 2, 1),    # 13.9, unsplit 13.2
+    (7, 5744, 5888, 4, 1),    # 10.2, two splits 11.6
+    (5, 5136, 1728, 4, 1),    # 4.5, unsplit 6.1
+])
+def test_one_row_tile_plan_on_measured_shapes(pkg, M, N, K, form, ksplit):
+    from featherops_amd.kernel.hip import _lib
+
+    assert _any_m_plan(_lib.lib(), M, N, K) == (10, ksplit, form)
