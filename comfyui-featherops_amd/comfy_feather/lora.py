@@ -88,20 +88,35 @@ def lora_factors(x: torch.Tensor, weight_functions, cache: dict | None = None):
 
 def lora_layer_inputs(x: torch.Tensor, weight_functions, cache: dict | None = None):
     """lora_factors(x, ...) and the activations the GEMM should be given: (T, U, x'), or None.
-    For bf16 x of more than 48 rows the GEMM takes fp16 activations, so with at most 128
-    ranks x' is x.to(float16) from the down-projection's own pass over x (the small-M kernel
-    that serves fewer rows takes bf16); otherwise x' is x."""
+    Where the GEMM with a rank-R term takes fp16 activations only, a bf16 x with at most 128
+    ranks becomes x' = x.to(float16) in the down-projection's own pass over x, a launch less
+    (layer with M=40 N=2048 K=1024 rank 32: 21.4 -> 17.5 us eagerly, 12.6 -> 11.3 in a graph);
+    otherwise x' is x."""
     factors = _factor_matrices(x, weight_functions, cache)
     if factors is None:
         return None
     d, u = factors
-    if (x.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] > 48 and d.shape[0] <= 128 and x.is_cuda
+    if (x.dtype == torch.bfloat16 and x.dim() == 2 and d.shape[0] <= 128 and x.is_cuda
+            and not gemm_takes_bf16(x.shape[0], u.shape[0], x.shape[1], cache)
             and x.shape[1] % 16 == 0 and x.shape[1] < (1 << 22) and x.is_contiguous()
             and x.data_ptr() % 16 == 0 and d.data_ptr() % 16 == 0):
         _lib.load_torch_ops()
         t, x16 = torch.ops.feather_ops.lora_down_cast.default(x, d)
         return t, u, x16
     return lora_down(x, d), u, x
+
+
+def gemm_takes_bf16(M: int, N: int, K: int, cache: dict | None = None) -> bool:
+    """Whether the GEMM with a rank-R term serves this shape with bf16 activations as they are:
+    on the lean small-M kernel, so never above 32 rows; below, the library's plan says (kept in
+    `cache`, a call of 1.6 us)."""
+    if M > 32:
+        return False
+    known = {} if cache is None else cache.setdefault("takes_bf16", {})
+    takes = known.get((M, N, K))
+    if takes is None:
+        takes = known[(M, N, K)] = _lib.lib().feather_scaled_mm_any_m_smallm_form(M, N, K, 1) != 0
+    return takes
 
 
 def _factor_matrices(x: torch.Tensor, weight_functions, cache: dict | None):

@@ -201,3 +201,22 @@ def test_linear_with_lora_patches(cuda, pkg, m):
     d_f = (y_fused.reshape(m, N).double().cpu() - exact).norm().item()
     d_s = (y_sep.reshape(m, N).double().cpu() - exact).norm().item()
     assert d_f <= d_s * 1.05, (d_f, d_s)
+
+
+@pytest.mark.parametrize("M,N,K,fused_cast", [(16, 1024, 512, False), (8, 2048, 12288, True), (33, 1024, 512, True),
+                                              (48, 512, 1040, True), (333, 512, 256, True)])
+def test_layer_inputs_cast_with_the_down_projection(cuda, hk, pkg, M, N, K, fused_cast):
+    """bf16 activations of a LoRA layer: in fp16 from the down-projection's own pass wherever the GEMM takes
+    no bf16 ones, with the result bits of the bf16 call."""
+    from featherops_amd.comfy_feather import lora
+
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).bfloat16().to(cuda)
+    bp = (torch.randn(K // 16, N, 16, generator=g) * 0.1).to(torch.float8_e5m2).to(cuda)
+    wf, _ = make_patches(N, K, [16], g, device=cuda, dtype=torch.bfloat16)
+    t, u, x2 = lora.lora_layer_inputs(x, wf, {})
+    assert x2.dtype == (torch.float16 if fused_cast else torch.bfloat16)
+    assert torch.equal(x2, x.to(x2.dtype))
+    y = hk.scaled_mm_hip_any_m_lora(x2, bp, None, None, torch.bfloat16, t, u)
+    want = hk.scaled_mm_hip_any_m_lora(x, bp, None, None, torch.bfloat16, t, u)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
