@@ -119,6 +119,12 @@ size_t tile_workspace_bytes(int tile, int64_t M, int64_t N, int ksplit);
 // Launches a tile with the given K split; ksplit > 1 needs tile_workspace_bytes() of
 // workspace (same contract as launch_smallm_kernel's).
 bool launch_tile(int tile, const MmArgs& p, int ksplit, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// Whether launch_tile runs a split-K tile on one group of waves, 64 K a stage, instead of two
+// groups (calls without a rank-R term): see launch_short.
+inline bool short_k_tile(int tile, int64_t K, int ksplit) {
+    return (tile == kLdsSk64x64 || tile == kLdsSk64x128 || tile == kLdsSk32x128) && ksplit == 1 && K % 64 == 0 && K <= 1024;
+}
+bool launch_short(int tile, const MmArgs& p, hipStream_t stream);
 int lds_pipe_env();  // FEATHEROPS_LDS_PIPE (1 unless set)
 bool launch_mid(int tile, const MmArgs& p, int ksplit, float* partials, uint32_t* counters, hipStream_t stream);
 

@@ -108,6 +108,7 @@ bool launch_tile(int tile, const MmArgs& p, int ksplit, void* workspace, size_t 
         partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kWorkspaceCounterBytes);
     }
     if (tile >= kMid32x64) return launch_mid(tile, p, ksplit, partials, counters, stream);
+    if (p.lora_dtype == 0 && short_k_tile(tile, p.K, ksplit)) return launch_short(tile, p, stream);
     if (tile == kLdsSk64x64 || tile == kLdsSk64x128 || tile == kLdsSk32x128)
         return launch_lds_pipe<1>(tile, p, stream, ksplit, partials, counters);
     return ksplit == 1 && launch_lds_kernel(tile, p, stream);

@@ -27,4 +27,20 @@ bool launch_mid(int tile, const MmArgs& p, int ksplit, float* partials, uint32_t
     }
 }
 
+// The split-K tiles unsplit on a short K: one group of 1 x 4 waves, a stage of 64 K, two
+// workgroups per CU past one round. Two groups with a stage of 128 K have half the stages to
+// fill their ring with and an exchange of sums at the end, about 0.7 us that a short K does not
+// earn back. us with the weight in HBM, two groups -> one: 64 x 64 M=260 N=3072 K=128 4.2 -> 3.5, K=320 5.0 ->
+// 4.2, K=640 5.5 -> 4.9, K=1024 6.2 -> 5.8; 64 x 128 M=600 N=3072 K=320 6.2 -> 5.2, K=768
+// 7.2 -> 6.9, K=1024 7.8 -> 7.7; 32 x 128 M=64 N=7168 K=512 5.0 -> 4.5. From K = 1280 on 64 x 128 loses
+// (8.5 vs 8.6), from 2048 on all do (64 x 64 with the weight in the MALL 9.3 vs 9.6).
+bool launch_short(int tile, const MmArgs& p, hipStream_t stream) {
+    switch (tile) {
+        case kLdsSk64x64: return launch_lds<64, 64, 1, 4, 1, 5>(p, stream);
+        case kLdsSk64x128: return launch_lds<64, 128, 1, 4, 1, 5>(p, stream);
+        case kLdsSk32x128: return launch_lds<32, 128, 1, 4, 1, 5>(p, stream);
+        default: return false;
+    }
+}
+
 }  // namespace feather

@@ -45,6 +45,15 @@ constexpr TileCost kTiles[] = {
     {kTail128x256, 128, 256, 1, true, 6.00, 0.501, 0.126, 7.20, 0, 0},
 };
 
+// The same for the split-K tiles' short form (short_k_tile): 136 shapes with the weight in
+// HBM, 3-4% rms, up to two workgroups per CU, which share it. Past those every workgroup's
+// epilogue counts and larger tiles win (M=777 N=4928 K=64 7.5 us on 64 x 64, 6.4 on 128 x 192).
+constexpr TileCost kShortTiles[] = {
+    {kLdsSk32x128, 32, 128, 1, false, 3.22, 0.156, 0.021, 0.3, 0, 0},
+    {kLdsSk64x64, 64, 64, 1, false, 3.16, 0.138, 0.041, 0.3, 0, 0},
+    {kLdsSk64x128, 64, 128, 1, false, 3.66, 0.216, 0.053, 1.0, 0, 0},
+};
+
 constexpr int kMaxSplit = 16;
 // Partial tiles of a split (a workspace that callers keep per stream)
 constexpr size_t kMaxSplitBytes = size_t(15) << 20;
@@ -97,10 +106,10 @@ SmallmChoice smallm_choice(int64_t M, int64_t N, int64_t K, int cus, bool lora, 
         if (us < best_us) best_us = us, best = {1, ks};
     };
     if (K % 64 == 0) {
-        // the lean kernel, two workgroups per CU (134 shapes, 6.3% rms); a short K on more than two
-        // rounds of strips is the tiles' (M=26 N=13696 K=384 5.5 vs 4.5 us)
+        // the lean kernel, two workgroups per CU (134 shapes, 6.3% rms); a fourth round of strips is
+        // the tiles', a third on a short K too (M=26 N=12736 K=768 6.9 vs 5.7 us, N=9968 K=384 4.6 vs 4.1)
         const double rounds = static_cast<double>(ceil_div(strips, cus));
-        if ((strips <= 2 * cus || K >= 512) && (!lora || is_lean(smallm_form(M, N, K, cus, 1, 1))))
+        if ((strips <= 2 * cus || (strips <= 3 * cus && K >= 512)) && (!lora || is_lean(smallm_form(M, N, K, cus, 1, 1))))
             offer(1, 1.89 + 0.484 * rounds + (0.0017 + 0.0011 * m + 0.085 * a) * rounds * nst + 0.156 * mb, slack);
     } else if (strips <= cus) {
         // the general kernel on 16-column strips (105 shapes, 6% rms)
@@ -123,6 +132,12 @@ SmallmChoice smallm_choice(int64_t M, int64_t N, int64_t K, int cus, bool lora, 
 
 const TileCost* tile_cost(int tile) {
     for (const TileCost& t : kTiles)
+        if (t.tile == tile) return &t;
+    return nullptr;
+}
+
+const TileCost* short_cost(int tile) {
+    for (const TileCost& t : kShortTiles)
         if (t.tile == tile) return &t;
     return nullptr;
 }
@@ -156,7 +171,9 @@ MmPlan make_plan(int64_t M, int64_t N, int64_t K, int cus, bool lora) {
                 if (tile_workspace_bytes(t.tile, M, N, ks) > kMaxSplitBytes) break;
             }
             last = ceil_div(stages, ks);
-            const double us = cost_us(t, tiles, stages, ks, cus);
+            const TileCost* const brief =
+                !lora && tiles <= 2 * cus && short_k_tile(t.tile, K, ks) ? short_cost(t.tile) : nullptr;
+            const double us = brief ? cost_us(*brief, tiles, ceil_div(K, 64), 1, cus) : cost_us(t, tiles, stages, ks, cus);
             if (us < best_us) {
                 best_us = us;
                 best.tile = t.tile;

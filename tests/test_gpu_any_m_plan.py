@@ -1,4 +1,4 @@
-"""The any-M entry's planned tiles (32 x 64 up to 128 x 256, two K groups, K splits, any K): one
+"""The any-M entry's planned tiles (32 x 64 up to 128 x 256, one and two K groups, K splits, any K): one
 shape per tile and K remainder, whole outputs against a float64 evaluation on the device, under the
 gate of gpu_util (fp32 sums in another order, two roundings to the output type)."""
 
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 # (M, N, K, kernel id, K splits > 1): K a multiple of 128, of 64 only, of 16 only, below one stage
 CASES = [
-    (63, 224, 128, 40, False), (77, 128, 64, 40, False), (63, 240, 16, 40, False), (65, 256, 112, 40, False),
+    (63, 224, 1152, 40, False), (77, 128, 1088, 40, False), (63, 240, 16, 40, False), (65, 256, 112, 40, False),
     (33, 128, 2480, 40, True), (48, 128, 2304, 40, True),
     (130, 5488, 128, 34, False), (130, 5664, 1232, 34, False), (17, 5456, 5648, 34, True),
     (191, 5024, 432, 30, False), (333, 1712, 3904, 30, False), (33, 2864, 4464, 30, True),
@@ -22,10 +22,15 @@ CASES = [
     (333, 5504, 1264, 42, False), (333, 5408, 1728, 42, False), (200, 4640, 5520, 42, True),
     (500, 4384, 2352, 43, False), (500, 4416, 2368, 43, False), (200, 5504, 4528, 43, True),
     (2000, 4224, 80, 44, False), (1003, 4304, 896, 44, False), (777, 5056, 4880, 44, False),
-    (200, 6112, 16, 45, False), (1003, 1632, 128, 45, False), (777, 4064, 2704, 45, False),
-    (777, 4688, 16, 46, False), (777, 4928, 64, 46, False), (1300, 3536, 2096, 46, False),
+    (200, 6112, 16, 45, False), (500, 5392, 128, 45, False), (777, 4064, 2704, 45, False),
+    (777, 4688, 16, 46, False), (777, 5104, 64, 46, False), (1300, 3536, 2096, 46, False),
     (2000, 3088, 16, 47, False), (1300, 4576, 48, 47, False), (2000, 3712, 4528, 47, False),
     (1500, 4592, 1040, 47, False),
+    # the split-K tiles on one group of waves (unsplit, K % 64 == 0 up to 1024): one stage of 64 K, fewer than
+    # the ring's five, as many, one more, the longest; one round of workgroups and two
+    (77, 128, 64, 30, False), (63, 224, 128, 30, False), (191, 5056, 320, 30, False), (97, 5040, 384, 30, False),
+    (1003, 1632, 128, 30, False), (777, 4928, 64, 31, False), (200, 5952, 384, 31, False), (1578, 2544, 832, 31, False),
+    (130, 5488, 1024, 34, False), (199, 8256, 192, 34, False),
 ]
 
 
