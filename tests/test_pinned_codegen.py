@@ -26,6 +26,9 @@ sys.path.insert(0, str(REPO))
 # the pinned tiles: default schedule (5th template argument 1), wave tiles of at least 64 x 64
 PINNED = r"scaled_mm_lds_kernelILi(256ELi256ELi4ELi2|256ELi128ELi4ELi2|128ELi256ELi2ELi4|128ELi128ELi2ELi2|" \
          r"256ELi192ELi4ELi2|128ELi384ELi2ELi4)ELi1E"
+# ... and the same tile for any K (last template argument kTail: the loop body may zero part of a landed stage)
+ANY_K = r"scaled_mm_lds_kernelILi128ELi256ELi2ELi4ELi1ELb([01])ELb([01])ELi0E\S*ELb1EE"
+SOURCES = ("scaled_mm_lds.hip", "scaled_mm_mid.hip")
 
 
 @pytest.fixture(scope="module")
@@ -33,13 +36,15 @@ def bodies(tmp_path_factory):
     import __graft_entry__
 
     b = __graft_entry__.load_build_module()
-    out = tmp_path_factory.mktemp("asm") / "scaled_mm_lds.s"
-    cmd = [b._hipcc(), *b.HIP_FLAGS, "--cuda-device-only", "-S", str(b.CSRC / "scaled_mm_lds.hip"), "-o", str(out)]
-    r = subprocess.run(cmd, capture_output=True, text=True, timeout=900)
-    assert r.returncode == 0, r.stderr[-2000:]
+    outs = [tmp_path_factory.mktemp("asm") / (Path(src).stem + ".s") for src in SOURCES]
+    procs = [subprocess.Popen([b._hipcc(), *b.HIP_FLAGS, "--cuda-device-only", "-S", str(b.CSRC / src), "-o", str(out)],
+                              stderr=subprocess.PIPE, text=True) for src, out in zip(SOURCES, outs)]
+    for proc in procs:
+        err = proc.communicate(timeout=900)[1]
+        assert proc.returncode == 0, err[-2000:]
     found = {}
     name = None
-    for line in out.read_text().splitlines():
+    for line in (line for out in outs for line in out.read_text().splitlines()):
         m = re.match(r"^(_Z\S+):", line)
         if m:
             name = m.group(1) if re.search(PINNED, m.group(1)) else None
@@ -100,6 +105,8 @@ def _loops(body: list) -> list:
 def test_pinned_tiles_are_compiled(bodies):
     # 4 output/weight-format variants x (no LoRA + 2 LoRA kinds for e5m2) per tile; at least the six tiles
     assert len({re.search(PINNED, n).group(1) for n in bodies}) == 6, sorted(bodies)[:3]
+    # the any-K tile: both output types x both weight types
+    assert {m.groups() for m in (re.search(ANY_K, n) for n in bodies) if m} == {("0", "0"), ("0", "1"), ("1", "0"), ("1", "1")}
 
 
 def test_mfmas_in_place_and_accumulators_untouched_in_loops(bodies):

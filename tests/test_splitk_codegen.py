@@ -89,6 +89,9 @@ def _check_protocol(name: str, body: list) -> None:
     ("scaled_mm_smallm.hip", r"scaled_mm_smallm_kernel", 8),
     ("lora_down.hip", r"lora_down_kernel", 4),
     ("scaled_mm_lds.hip", r"scaled_mm_lds_kernelILi(64ELi64|64ELi128|32ELi128)E", 12),
+    # the planned tiles with two K groups of 1 x 4 waves (the others there are never launched with a K
+    # split and hold no protocol): five tiles x (four type combinations + a rank-R term for two outputs)
+    ("scaled_mm_mid.hip", r"scaled_mm_lds_kernelILi(32ELi64|96ELi64|96ELi128|64ELi192|96ELi192)ELi1ELi4E\S*ELi2ELb1EE", 28),
 ])
 def test_split_k_arrival_order_in_compiled_code(tmp_path, src, kernel_re, min_kernels):
     bodies = _bodies(_asm(tmp_path, src), kernel_re)
