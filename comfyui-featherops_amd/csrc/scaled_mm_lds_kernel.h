@@ -654,15 +654,33 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
         // MFMA steps read their fragments from LDS. Step kh covers ranks
         // [32 kh, 32 kh + 32): lane group lg reads chunk lg + 4 kh of T and U.
         // A 32-rank tail copies ranks [0, 32) only and runs step 0.
-        const uint32_t lt = lds_addr_of(sbuf0);
-        const uint32_t lu = lds_addr_of(sbuf1);
+        // kSlots chunks are in flight at a time where the ring has room (both factors in one
+        // stage buffer, or in two): their round trips would otherwise follow one another (us, one
+        // in flight -> kSlots, rank 1024: M=154 N=K=3072 23.8 -> 20.7, M=1000 41.6 -> 37.9, M=8
+        // N=2048 K=12288 23.6 -> 20.9, rank 512 18.1 -> 17.3; up to 64 ranks the same; as many as
+        // the ring has stages, six there: 21.5).
+        constexpr bool kOneBuf = kStage >= (BM + BN) * 128;
+        constexpr int kSlots = kOneBuf ? 3 : kStages >= 4 ? 2 : 1;
+        auto slot_t = [&](int slot) -> uint32_t {
+            if constexpr (kOneBuf) return slot == 0 ? lds_addr_of(sbuf0) : slot == 1 ? lds_addr_of(sbuf1) : lds_addr_of(sbuf2);
+            else return slot == 0 ? lds_addr_of(sbuf0) : lds_addr_of(sbuf2);
+        };
+        auto slot_u = [&](int slot) -> uint32_t {
+            if constexpr (kOneBuf) return slot_t(slot) + BM * 128;
+            else return slot == 0 ? lds_addr_of(sbuf1) : lds_addr_of(sbufx);
+        };
         constexpr int kTInst = BM / 8;  // 1 KB copies: 8 rows of 64 ranks
         constexpr int kUInst = BN / 8;
-        for (int r0 = 0; r0 < lora_rank; r0 += 64) {
+        // the same number for every wave, so that the wait counts are constants: surplus
+        // ones repeat the last copy
+        constexpr int kPerWave = (kTInst + kUInst + kWaves - 1) / kWaves;
+        const int chunks = (lora_rank + 63) / 64;
+        auto issue_chunk = [&](int ch, int slot) {
+            const int r0 = ch * 64;
             const bool rtail = lora_rank - r0 < 64;
-            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of the buffers are done
-            stage_barrier();                      // and every other wave's
-            for (int j = wave; j < kTInst + kUInst; j += kWaves) {
+#pragma unroll
+            for (int i = 0; i < kPerWave; ++i) {
+                const int j = i * kWaves + wave < kTInst + kUInst ? i * kWaves + wave : kTInst + kUInst - 1;
                 const bool is_t = j < kTInst;
                 const int jj = is_t ? j : j - kTInst;
                 const int row = jj * 8 + (lane >> 3);
@@ -670,11 +688,22 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
                 if (rtail && c >= 4) c -= 4;  // past the rank: a valid chunk, never read
                 const int grow = is_t ? (m0 + row < M ? m0 + row : M - 1) : (n0 + row < N ? n0 + row : N - 1);
                 dma16_lds(is_t ? lora_t : lora_u, static_cast<uint32_t>((grow * lora_rank + r0 + 8 * c) * 2),
-                          (is_t ? lt : lu) + jj * 1024);
+                          (is_t ? slot_t(slot) : slot_u(slot)) + jj * 1024);
             }
-            wait_vmcnt<0>();
+        };
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of the buffers are done
+        stage_barrier();                      // and every other wave's
+#pragma unroll
+        for (int i = 0; i < kSlots; ++i)
+            if (i < chunks) issue_chunk(i, i);
+        int slot = 0;
+        for (int ch = 0; ch < chunks; ++ch) {
+            // chunk ch has landed once only the kSlots - 1 after it are outstanding
+            if (ch + kSlots <= chunks) wait_vmcnt<(kSlots - 1) * kPerWave>();
+            else wait_vmcnt<0>();
             stage_barrier();
-            for (int kh = 0; kh < (rtail ? 1 : 2); ++kh) {
+            const uint32_t lt = slot_t(slot), lu = slot_u(slot);
+            for (int kh = 0; kh < (lora_rank - ch * 64 < 64 ? 1 : 2); ++kh) {
                 uint4 tf[RME], uf[RN];
 #pragma unroll
                 for (int rm = 0; rm < RME; ++rm) {
@@ -696,6 +725,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
                             dst[rm][rn] = mfma16x16x32_bf16(uf[rn], tf[rm], dst[rm][rn]);
                     }
             }
+            if (ch + kSlots < chunks) {
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // the slot's readers are done
+                stage_barrier();
+                issue_chunk(ch + kSlots, slot);
+            }
+            slot = slot + 1 < kSlots ? slot + 1 : 0;
         }
     };
     if constexpr (kLora == 1 || kLora == 2) {

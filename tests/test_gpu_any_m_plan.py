@@ -78,13 +78,7 @@ LORA_SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("out_dtype,f_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
-                                               (torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)])
-@pytest.mark.parametrize("M,N,K", LORA_SHAPES)
-def test_planned_tile_lora(cuda, hk, M, N, K, out_dtype, f_dtype):
-    """The rank-R term on every planned tile, against the whole output in float64 with the term in the
-    accumulator (tuple route on a large tile) or rounded and added to the result (every other)."""
-    R = 32 * (1 + (M + N // 16) % 5)
+def _check_lora(cuda, hk, M, N, K, R, out_dtype, f_dtype):
     g = torch.Generator(device=cuda).manual_seed(M + N + K + 1)
     a = torch.randn(M, K, generator=g, device=cuda).half()
     w = torch.randn(N, K, generator=g, device=cuda) * 0.02
@@ -109,3 +103,27 @@ def test_planned_tile_lora(cuda, hk, M, N, K, out_dtype, f_dtype):
     yb = hk.scaled_mm_hip_any_m_lora(ab, bp, s, bias, out_dtype, t, u)
     y16 = hk.scaled_mm_hip_any_m_lora(ab.half(), bp, s, bias, out_dtype, t, u)
     assert torch.equal(yb.view(torch.int16), y16.view(torch.int16))
+
+
+@pytest.mark.parametrize("out_dtype,f_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
+                                               (torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)])
+@pytest.mark.parametrize("M,N,K", LORA_SHAPES)
+def test_planned_tile_lora(cuda, hk, M, N, K, out_dtype, f_dtype):
+    """The rank-R term on every planned tile, against the whole output in float64 with the term in the
+    accumulator (tuple route on a large tile) or rounded and added to the result (every other)."""
+    _check_lora(cuda, hk, M, N, K, 32 * (1 + (M + N // 16) % 5), out_dtype, f_dtype)
+
+
+# the lean kernel (loads of 128 ranks in flight; one and two row tiles, one and two workgroups per CU), the tiles whose
+# stage buffer holds 64 ranks of both factors (three of those in flight), those that need two (two in flight) and a
+# large tile (one)
+MANY_RANK_SHAPES = [(5, 528, 512), (16, 4112, 512), (31, 1040, 1024), (63, 224, 128), (33, 128, 2480), (130, 5488, 128),
+                    (333, 1712, 3904), (333, 2976, 1664), (97, 4160, 3984), (333, 5408, 1728), (500, 4416, 2368),
+                    (777, 5056, 4880), (777, 4064, 2704), (777, 4928, 64), (2000, 6160, 128)]
+
+
+@pytest.mark.parametrize("R", [96, 192, 224, 256, 320, 416, 1024])
+@pytest.mark.parametrize("M,N,K", MANY_RANK_SHAPES)
+def test_planned_tile_lora_many_ranks(cuda, hk, M, N, K, R):
+    """Ranks around every number of 64-rank chunks in flight, stacks of several hundred among them."""
+    _check_lora(cuda, hk, M, N, K, R, torch.bfloat16, torch.bfloat16)
