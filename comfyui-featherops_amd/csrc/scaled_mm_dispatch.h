@@ -91,7 +91,6 @@ struct SplitKPlan {
     int kernel_id;          // 0: not applicable
     int ksplit;
     int tiles;
-    size_t counter_bytes;   // the fixed counter region (kWorkspaceCounterBytes) when ksplit > 1
     size_t workspace_bytes; // counter region + ksplit fp32 partial tiles per output tile
 };
 SplitKPlan lds_splitk_plan(int64_t M, int64_t N, int64_t K, int target);

@@ -94,8 +94,7 @@ SplitKPlan lds_splitk_plan(int64_t M, int64_t N, int64_t K, int target) {
     pl.kernel_id = bm == 32 ? kLdsSk32x128 : bn == 128 ? kLdsSk64x128 : kLdsSk64x64;
     pl.ksplit = static_cast<int>(ks);
     pl.tiles = static_cast<int>(tiles);
-    pl.counter_bytes = ks > 1 ? kWorkspaceCounterBytes : 0;
-    pl.workspace_bytes = ks > 1 ? pl.counter_bytes + static_cast<size_t>(tiles) * ks * bm * bn * 4 : 0;
+    pl.workspace_bytes = ks > 1 ? kWorkspaceCounterBytes + static_cast<size_t>(tiles) * ks * bm * bn * 4 : 0;
     return pl;
 }
 

@@ -502,14 +502,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
         // Plain schedule: at the top of stage kt wait for its copies (issued
         // two stages earlier), barrier, issue stage kt + 2's copies into the
         // buffer stage kt - 1 used, then read and multiply both K halves.
+        static_assert(!kTail, "the plain schedule has no shifted last stage");
         auto no_hook = [](int) {};
         auto run_stage = [&](auto cur, int kt) {
             constexpr int c = decltype(cur)::value;
             using Free = std::integral_constant<int, (c + 2) % 3>;
             if (kt + 1 < nk) wait_vmcnt<kLoadsPerStage>();
             else wait_vmcnt<0>();
-            if constexpr (kTail)
-                if (tail && kt + 1 == nk) zero_tail(cur);
             stage_barrier();
             if (kt + 2 < nk) issue_stage(Free{}, stage_k(kt + 2, Near{}));
             uint4 braw[RN];
