@@ -7,6 +7,12 @@
 
 namespace feather {
 
+// Shape limits every kernel family relies on: the LDS kernels build per-lane copy offsets within a
+// tile in 32 bits, row * K * 2 over at most 256 rows (below 2^31) and (16-K group * N + column) * 16
+// over a stage's eight groups at most (unsigned, below 2^32; the kernel asserts both).
+constexpr int64_t kMaxK = int64_t{1} << 22;
+constexpr int64_t kMaxN = int64_t{1} << 25;
+
 struct MmArgs {
     const uint16_t* a;       // (M, K) fp16 (or bf16 when a_bf16), row-major
     const uint8_t* b;        // (K/16, N, 16) fp8 bytes

@@ -101,6 +101,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * kGroups) void scaled_mm_ld
     constexpr int RN = WTN / 16;
     static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be a multiple of 16");
     constexpr int kSK = kBK * kGroups;  // K per stage
+    // the 32-bit copy offsets a_off and b_off below (see kMaxK, kMaxN)
+    static_assert(int64_t{BM} * kMaxK * 2 <= int64_t{1} << 31 && int64_t{kSK / 16} * kMaxN * 16 <= int64_t{1} << 32,
+                  "copy offsets fit 32 bits");
     constexpr int kASub = BM * kBK * 2;  // one group's share of a stage
     constexpr int kBSub = BN * kBK;
     constexpr int kAStage = kASub * kGroups;
