@@ -484,8 +484,8 @@ def bench_lora(dev, hk, g) -> dict:
     wf = [SimpleNamespace(patches={"w": [(1.0, SimpleNamespace(weights=(up, down, float(R), None)), 1.0)]}, key="w")]
 
     def fused(_i):
-        t, u = lora.lora_factors(x, wf)
-        return hk.scaled_mm_hip_any_m_lora(x, bp, s, bias, torch.bfloat16, t, u)
+        t, u, x16 = lora.lora_layer_inputs(x, wf)  # what Linear.forward runs
+        return hk.scaled_mm_hip_any_m_lora(x16, bp, s, bias, torch.bfloat16, t, u)
 
     def separate(_i):
         y = hk.scaled_mm_hip_any_m(x, bp, s, bias, torch.bfloat16)
