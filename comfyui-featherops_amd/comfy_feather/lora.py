@@ -82,7 +82,7 @@ def lora_factors(x: torch.Tensor, weight_functions, cache: dict | None = None):
     factors = _factor_matrices(x, weight_functions, cache)
     if factors is None:
         return None
-    d, u = factors
+    d, u, _ = factors
     return lora_down(x, d), u
 
 
@@ -95,31 +95,28 @@ def lora_layer_inputs(x: torch.Tensor, weight_functions, cache: dict | None = No
     factors = _factor_matrices(x, weight_functions, cache)
     if factors is None:
         return None
-    d, u = factors
-    if (x.dtype == torch.bfloat16 and x.dim() == 2 and d.shape[0] <= 128 and x.is_cuda
-            and not gemm_takes_bf16(x.shape[0], u.shape[0], x.shape[1], cache)
-            and x.shape[1] % 16 == 0 and x.shape[1] < (1 << 22) and x.is_contiguous()
-            and x.data_ptr() % 16 == 0 and d.data_ptr() % 16 == 0):
-        _lib.load_torch_ops()
-        t, x16 = torch.ops.feather_ops.lora_down_cast.default(x, d)
-        return t, u, x16
+    d, u, takes_bf16 = factors
+    if x.dtype == torch.bfloat16 and x.dim() == 2:
+        m, k = x.shape
+        takes = takes_bf16.get(m) if m <= 32 else False  # (a call of the library takes 1.6 us)
+        if takes is None:
+            takes = takes_bf16[m] = gemm_takes_bf16(m, u.shape[0], k)
+        if (not takes and d.shape[0] <= 128 and x.is_cuda and k % 16 == 0 and k < (1 << 22) and x.is_contiguous()
+                and x.data_ptr() % 16 == 0 and d.data_ptr() % 16 == 0):
+            _lib.load_torch_ops()
+            t, x16 = torch.ops.feather_ops.lora_down_cast.default(x, d)
+            return t, u, x16
     return lora_down(x, d), u, x
 
 
-def gemm_takes_bf16(M: int, N: int, K: int, cache: dict | None = None) -> bool:
+def gemm_takes_bf16(M: int, N: int, K: int) -> bool:
     """Whether the GEMM with a rank-R term serves this shape with bf16 activations as they are:
-    on the lean small-M kernel, so never above 32 rows; below, the library's plan says (kept in
-    `cache`, a call of 1.6 us)."""
-    if M > 32:
-        return False
-    known = {} if cache is None else cache.setdefault("takes_bf16", {})
-    takes = known.get((M, N, K))
-    if takes is None:
-        takes = known[(M, N, K)] = _lib.lib().feather_scaled_mm_any_m_smallm_form(M, N, K, 1) != 0
-    return takes
+    on the lean small-M kernel, so never above 32 rows; below, the library's plan says."""
+    return M <= 32 and _lib.lib().feather_scaled_mm_any_m_smallm_form(M, N, K, 1) != 0
 
 
 def _factor_matrices(x: torch.Tensor, weight_functions, cache: dict | None):
+    """(D, U, what gemm_takes_bf16 said for these factors by row count) or None, see lora_factors."""
     if x.dtype not in (torch.float16, torch.bfloat16):
         return None
     patches = _basic_patches(weight_functions)
@@ -127,16 +124,18 @@ def _factor_matrices(x: torch.Tensor, weight_functions, cache: dict | None):
         return None
     if cache is None:
         d, u = _stacked_factors(x, patches)
+        takes_bf16 = {}
     else:
         key = (x.dtype, x.device, tuple((id(dn), dn._version, id(up), up._version, float(sc))
                                         for dn, up, sc in patches))
         hit = cache.get("entry")
         if hit is not None and hit[0] == key:
-            d, u = hit[2], hit[3]
+            d, u, takes_bf16 = hit[2], hit[3], hit[4]
         else:
             d, u = _stacked_factors(x, patches)
-            cache["entry"] = (key, [(dn, up) for dn, up, _ in patches], d, u)
-    return d, u
+            takes_bf16 = {}
+            cache["entry"] = (key, [(dn, up) for dn, up, _ in patches], d, u, takes_bf16)
+    return d, u, takes_bf16
 
 
 def lora_down(x: torch.Tensor, d: torch.Tensor) -> torch.Tensor:

@@ -101,16 +101,14 @@ def test_factor_cache_reuse_and_invalidation(lora):
 
 def test_gemm_takes_bf16_as_the_plan_does(lora):
     """bf16 activations go to the GEMM as they are only where its plan with a rank-R term is the lean small-M
-    kernel: never above 32 rows, and below not on a tile; the answer is kept per shape in the layer's cache."""
+    kernel: never above 32 rows, and below not on a tile."""
     from featherops_amd.kernel.hip import _lib
 
-    L, cache = _lib.lib(), {}
+    L = _lib.lib()
     seen = set()
     for M in (1, 8, 16, 17, 24, 32, 33, 40, 48, 49, 4096):
         for N, K in ((2048, 12288), (4096, 4096), (12288, 3072), (1040, 1040), (512, 4096)):
-            takes = lora.gemm_takes_bf16(M, N, K, cache)
+            takes = lora.gemm_takes_bf16(M, N, K)
             assert takes == (L.feather_scaled_mm_any_m_smallm_form(M, N, K, 1) in (3, 4)), (M, N, K)
-            assert takes == lora.gemm_takes_bf16(M, N, K, cache) == lora.gemm_takes_bf16(M, N, K)
             seen.add((M > 32, takes))
     assert seen == {(False, False), (False, True), (True, False)}
-    assert not any(M > 32 for M, _, _ in cache["takes_bf16"])
