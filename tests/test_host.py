@@ -442,6 +442,8 @@ def test_small_m_plan_and_launch_share_one_form(pkg):
     (26, 944, 10944, True, True),   # 9.0 (bf16 9.4), unsplit 14.2, tile 9.3 (bf16 12.0)
     (24, 4480, 3328, True, False),  # lean 10.0 (bf16 10.4), wide strips 11.7, tile 8.1 (bf16 11)
     (30, 7488, 1024, True, False),  # lean 4.6 (bf16 5.1), wide strips 5.9 (bf16 8.1), tile 5.2 (bf16 7.4)
+    (29, 3184, 6080, True, False),  # lean 10.6 (bf16 10.6), tile 9.5 (bf16 12.4)
+    (27, 3712, 7936, False, False),  # lean 13.0 (bf16 13.2), tile 10.7 (bf16 13.9)
     (30, 4992, 3152, False, False),  # wide strips 12.8, tile 8.7
     (48, 2976, 2016, False, False),  # 16-column strips 6.8 (bf16 9.1), tile 6.5 (bf16 8.9)
     (47, 1488, 1792, False, False),  # 7.7 (bf16 10.0), tile 5.9 (bf16 8.4)
