@@ -25,13 +25,16 @@
 //     Two groups of four waves now share a stage of 128 K, each multiplying its
 //     own 64 for the whole tile, so that every SIMD has two waves and there is one
 //     barrier per 128 K; the groups' sums meet once, through LDS, after the
-//     last stage. Back to back, one group on a five- or six-stage ring -> two:
-//     M=154 N=10240 K=4096 21.3 -> 17.3 us, M=333 N=K=3072 15.7 -> 13.2, M=256
-//     N=K=3072 11.7 -> 9.9, M=512 N=3072 K=12288 47.7 -> 42.4, M=128 N=K=5120
-//     14.5 -> 13.3, M=77 N=K=4096 11.5 -> 9.6, M=64 N=13824 K=5120 22.1 ->
-//     20.6, M=256 N=K=1024 5.5 -> 5.3. Four groups on 64 x 64 (16 waves): 10.6
-//     at M=256 N=K=3072; 2 x 4 waves instead of two groups: 64 x 128 18.1 at
-//     M=154, and more LDS reads per MFMA;
+//     last stage. One group on a five- or six-stage ring -> two, back to back with
+//     the weights in the MALL: M=154 N=10240 K=4096 21.3 -> 17.3 us, M=333 N=K=3072
+//     15.7 -> 13.2, M=256 N=K=3072 11.7 -> 9.9, M=512 N=3072 K=12288 47.7 -> 42.4,
+//     M=128 N=K=5120 14.5 -> 13.3, M=77 N=K=4096 11.5 -> 9.6, M=64 N=13824 K=5120
+//     22.1 -> 20.6. With the weights from HBM the gain is smaller or none: M=600
+//     N=1024 K=3072 11.3 -> 9.6, M=260 N=K=3072 11.9 -> 11.1, M=130 N=7168 K=4096 17.7 ->
+//     17.0, but M=154 N=10240 K=4096 20.5 -> 21.4 and M=128 N=7296 K=4416 17.0 -> 17.4.
+//     An unsplit K up to 1024 stays on one group (launch_short). Four groups on
+//     64 x 64 (16 waves): 10.6 at M=256 N=K=3072 in the MALL; 2 x 4 waves instead of two
+//     groups: 64 x 128 18.1 at M=154, and more LDS reads per MFMA;
 //   * per stage, the K halves are processed one after the other (all M
 //     repeats of K half 0, then of K half 1), so only half of the widened B
 //     operands are live at a time;

@@ -268,8 +268,8 @@ at::Tensor scaled_mm_configured_meta(const at::Tensor& a, const at::Tensor& b_pr
 // the strengths are folded into T by the caller). T (M, R) and U (N, R) are
 // contiguous fp16 or bf16 with R % 32 == 0. The GEMM's epilogue adds the term: to the
 // scaled fp32 accumulator where the tuple route takes a large LDS tile, else to the
-// finished result in the output type. Where no kernel does (e4m3fn weights, K % 64 != 0
-// on wide grids) the GEMM runs as scaled_mm_any_m and a second pass adds the term to C.
+// finished result in the output type. Where no kernel does (e4m3fn weights, the 128 x 256
+// any-K tile) the GEMM runs as scaled_mm_any_m and a second pass adds the term to C.
 at::Tensor scaled_mm_any_m_lora(const at::Tensor& a, const at::Tensor& b_prepacked,
                                 const std::optional<at::Tensor>& scale, const std::optional<at::Tensor>& bias,
                                 at::ScalarType out_dtype, const at::Tensor& lora_t, const at::Tensor& lora_u) {

@@ -328,8 +328,10 @@ def scaled_mm_hip_any_m_lora(a, b_prepacked, scale, bias, out_dtype, lora_t, lor
     lora_t (M, R); lora_u is (N, R); both contiguous fp16 or bf16, R % 32 == 0.
     Where any_m_config names a large LDS tile the term joins the fp32
     accumulator before the output rounding; elsewhere it is added to the
-    finished result in the output type, in the epilogue of the kernels that
-    take it, else (e4m3fn weights, wide or split small-M strips) by a pass over C."""
+    finished result in the output type, in the epilogue of the kernel that the plan
+    of a call with such a term takes: the lean small-M kernel or a tile (where the plain
+    call runs on wide or split small-M strips the sum's order differs from it). By a pass over
+    C for e4m3fn weights and on the 128 x 256 any-K tile."""
     return torch.ops.feather_ops.scaled_mm_any_m_lora.default(a, b_prepacked, scale, bias, out_dtype, lora_t, lora_u)
 
 

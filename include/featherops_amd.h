@@ -135,8 +135,8 @@ bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b
  * tile the term joins the scaled fp32 accumulator; elsewhere it is rounded to the
  * factors' type and to the output type and added to the finished result in the output
  * type, as a separate pass would. Returns false and launches nothing where no kernel
- * adds the term (e4m3fn weights; bf16 activations beyond the small-M kernel; K % 64
- * != 0 on the widest grids). Workspace: the size below, the contract of
+ * adds the term (e4m3fn weights; bf16 activations beyond the lean small-M kernel; K % 64
+ * != 0 where the plan takes the 128 x 256 tile). Workspace: the size below, the contract of
  * feather_launch_scaled_mm_ws.
  */
 size_t feather_scaled_mm_any_m_lora_workspace_size(int64_t M, int64_t N, int64_t K);
