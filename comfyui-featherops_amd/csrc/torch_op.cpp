@@ -41,9 +41,10 @@ namespace {
 // gets that buffer (its address would stay in the graph after a replacement has freed it) and an
 // eager call none made under capture (its zero fill runs with the graph's replays only): the
 // calls of one capture on one stream share a buffer allocated and zeroed inside that capture,
-// whose memory torch keeps for the graph, so graphs share nothing with each other either. The
-// caller holds the returned tensor until its kernels are enqueued: a call of another thread on
-// this stream may replace the buffer meanwhile.
+// whose memory torch keeps for the graph, so graphs share nothing with each other either (the
+// tensor itself is held until the stream's next capture, for one that was not begun through
+// torch). The caller holds the returned tensor until its kernels are enqueued: a call of
+// another thread on this stream may replace the buffer meanwhile.
 at::Tensor workspace_for(const at::Device& dev, hipStream_t stream, size_t nbytes) {
     constexpr int64_t kCounterBytes = 65536;
     struct Buffers {
@@ -63,11 +64,11 @@ at::Tensor workspace_for(const at::Device& dev, hipStream_t stream, size_t nbyte
     const auto options = at::TensorOptions().dtype(at::kByte).device(dev);
     std::lock_guard<std::mutex> lock(mu);
     Buffers& b = pool[{dev.index(), stream}];
-    if (!capturing || b.capture != id) b.captured.reset();  // a capture that has ended: the graph's memory alone
     if (!capturing) {
         if (!b.eager.defined() || static_cast<size_t>(b.eager.numel()) < nbytes) b.eager = at::zeros({n}, options);
         return b.eager;
     }
+    if (b.capture != id) b.captured.reset();  // of a capture that has ended: its graph's memory alone
     b.capture = id;
     if (!b.captured.defined() || static_cast<size_t>(b.captured.numel()) < nbytes) {
         b.captured = at::empty({n}, options);
