@@ -8,7 +8,7 @@ import ctypes
 import pytest
 import torch
 
-from gpu_util import assert_gemm_close_dev, lib, torch_ref_dev
+from gpu_util import assert_gemm_close_dev, lib, stream, torch_ref_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -68,3 +68,37 @@ def test_small_m_pair_lora(cuda, hk, M, N, K, R):
     # two bf16 roundings: of the term (relative 2^-9) and of the sum
     bound = 2.0**-8 * ((t.double() @ u.double().T).abs() + want.abs()) + 1e-6
     assert ((y.double() - want).abs() <= bound).all()
+
+
+STRIPS, WIDE = 1, 2
+
+
+@pytest.mark.parametrize("M,N,K,form,split", [
+    (31, 640, 9696, STRIPS, True), (17, 272, 11024, STRIPS, True), (32, 560, 8256, STRIPS, True),
+    (26, 944, 10944, STRIPS, True), (29, 2736, 1824, STRIPS, False), (23, 9520, 752, WIDE, False),
+    (41, 3616, 1056, STRIPS, False), (48, 4080, 400, STRIPS, False)])
+def test_small_m_planned_forms(cuda, hk, M, N, K, form, split):
+    """The other forms of 17..48 rows that the any-M plan hands to the launch (strip width and K split): whole
+    outputs against float64, bf16 activations as their fp16 cast, and through the C entry without a workspace
+    (K then split inside the workgroups only)."""
+    ks = ctypes.c_int()
+    assert lib().feather_scaled_mm_any_m_plan(M, N, K, ctypes.byref(ks)) == 10 and (ks.value > 1) == split
+    assert lib().feather_scaled_mm_any_m_smallm_form(M, N, K, 0) == form
+    assert (lib().feather_scaled_mm_any_m_workspace_size(M, N, K) > 0) == split
+    print("small-M form", M, N, K, form, ks.value, flush=True)
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    ab = torch.randn(M, K, generator=g, device=cuda).bfloat16()
+    a = ab.half()
+    w = torch.randn(N, K, generator=g, device=cuda) * 0.02
+    s = (w.abs().max() / 57344.0).float().reshape(1)
+    bp = (w / s).to(torch.float8_e5m2).view(N, K // 16, 16).permute(1, 0, 2).contiguous()
+    bias = (torch.randn(N, generator=g, device=cuda) * 0.1).half()
+    ref = torch_ref_dev(a, bp, s, bias, torch.float16)
+    y = hk.scaled_mm_hip_any_m(a, bp, s, bias, torch.float16)
+    assert_gemm_close_dev(y, ref, torch.float16, f"{M}x{N}x{K}")
+    for x in (ab, a):  # again, and with bf16 activations
+        assert torch.equal(y.view(torch.int16), hk.scaled_mm_hip_any_m(x, bp, s, bias, torch.float16).view(torch.int16))
+    c = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+    assert lib().feather_launch_scaled_mm_any_m(a.data_ptr(), 0, bp.data_ptr(), s.data_ptr(), bias.data_ptr(), c.data_ptr(),
+                                                M, N, K, 1, 1, 1, 0, None, 0, stream(cuda))
+    assert_gemm_close_dev(c, ref, torch.float16, f"{M}x{N}x{K} without a workspace")
