@@ -15,10 +15,19 @@ Two forms:
     in its epilogue, so C is written once.
 """
 
+import functools
+
 import torch
 import torch.nn.functional as F
 
 from ..kernel.hip import _lib
+
+
+@functools.cache
+def _op(name: str):
+    """torch.ops.feather_ops.<name>, the library loaded."""
+    _lib.load_torch_ops()
+    return getattr(torch.ops.feather_ops, name).default
 
 
 def _basic_patches(weight_functions):
@@ -103,8 +112,7 @@ def lora_layer_inputs(x: torch.Tensor, weight_functions, cache: dict | None = No
             takes = takes_bf16[m] = gemm_takes_bf16(m, u.shape[0], k)
         if (not takes and d.shape[0] <= 128 and x.is_cuda and k % 16 == 0 and k < (1 << 22) and x.is_contiguous()
                 and x.data_ptr() % 16 == 0 and d.data_ptr() % 16 == 0):
-            _lib.load_torch_ops()
-            t, x16 = torch.ops.feather_ops.lora_down_cast.default(x, d)
+            t, x16 = _op("lora_down_cast")(x, d)
             return t, u, x16
     return lora_down(x, d), u, x
 
@@ -144,13 +152,12 @@ def lora_down(x: torch.Tensor, d: torch.Tensor) -> torch.Tensor:
     refuse the operands: x not on the GPU, K not a multiple of 8 (16-byte row loads), ranks not a
     multiple of 32 or above 65536, K >= 2^24, or a storage offset that leaves x or d off a
     16-byte boundary."""
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     K, R = x2.shape[1], d.shape[0]
     if x2.is_cuda and K % 8 == 0 and R % 32 == 0 and R <= 65536 and K < (1 << 24):
         x2 = x2.contiguous()
         dc = d.contiguous()
         if x2.data_ptr() % 16 == 0 and dc.data_ptr() % 16 == 0:
-            _lib.load_torch_ops()
-            t = torch.ops.feather_ops.lora_down.default(x2, dc)
-            return t.reshape(*x.shape[:-1], R)
+            t = _op("lora_down")(x2, dc)
+            return t if x.dim() == 2 else t.reshape(*x.shape[:-1], R)
     return F.linear(x, d).contiguous()
