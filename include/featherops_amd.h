@@ -112,17 +112,16 @@ bool feather_launch_scaled_mm_ex(const void* a, int a_dtype, const uint8_t* b_pr
  * it. With less than feather_scaled_mm_any_m_workspace_size() bytes of workspace
  * it runs without a K split; the workspace contract is
  * feather_launch_scaled_mm_ws's. The choice is the same for every type.
- * bf16 activations are served by the small-M kernel with e5m2 weights; where the
- * shape takes another kernel it returns false and launches nothing (the caller
- * converts A and calls again). No
- * counterpart in the reference.
+ * bf16 activations are served by the small-M forms named below with e5m2 weights;
+ * elsewhere it returns false and launches nothing (the caller converts A and calls
+ * again). No counterpart in the reference.
  */
 size_t feather_scaled_mm_any_m_workspace_size(int64_t M, int64_t N, int64_t K);
 /* The kernel id (csrc/scaled_mm_dispatch.h) that entry takes and, in *ksplit (may be NULL), its K split. */
 int feather_scaled_mm_any_m_plan(int64_t M, int64_t N, int64_t K, int* ksplit);
 /* The form of the small-M kernel it takes (lora: the entry with a rank-R term below): 0 another kernel, 1 16-column
  * strips, 2 wider strips, 3 the lean kernel, 4 the lean kernel with two workgroups per CU. Up to 32 rows, forms 1, 3
- * and 4 take bf16 activations. */
+ * and 4 take bf16 activations, up to 16 rows all of them. */
 int feather_scaled_mm_any_m_smallm_form(int64_t M, int64_t N, int64_t K, int lora);
 bool feather_launch_scaled_mm_any_m(const void* a, int a_dtype, const uint8_t* b_prepacked, const float* scale,
                                     const uint16_t* bias, uint16_t* c, int64_t M, int64_t N, int64_t K, int has_scale,
